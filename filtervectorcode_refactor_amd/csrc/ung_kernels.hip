@@ -4,14 +4,21 @@
 // the two form one translation unit.
 //
 // Path (one call = one "job list"):
-//   select  : fused distance tiles on the bf16 matrix cores -- every fp32 coordinate
-//             is split into bf16 hi + lo and each product is taken as hi*hi + hi*lo +
-//             lo*hi by three v_mfma_f32_32x32x16_bf16 passes (LDS-staged candidate
-//             panels, query rows held in registers and LDS at dp = 128) -- with
-//             per-row register queues in the epilogue: no distance matrix ever reaches
-//             HBM.  At the end of a work item the approximate (expansion-form) top-Lp
-//             of every query is written as a partial row with a bound that every
-//             candidate left out satisfies.
+//   select  : fused distance tiles on the matrix cores (LDS-staged candidate panels) with
+//             per-row queues in the epilogue: no distance matrix ever reaches HBM.  At the
+//             end of a work item the approximate (expansion-form) top-Lp of every query is
+//             written as a partial row with a bound that every candidate left out
+//             satisfies.  Operands:
+//               half  : every coordinate scaled by a power of two and rounded to fp16, one
+//                       v_mfma_f32_32x32x16_f16 product; the certificate carries the
+//                       largest rounding error the base set really has.  A third of the
+//                       matrix work and half the operand bytes of the split (cross select
+//                       1M x 128 14.2 -> 9.0 ms, 1M x 384 15.5 -> 8.5 ms, 2M x 768 160 ->
+//                       80 ms);
+//               split : bf16 hi + lo of every coordinate, products hi*hi + hi*lo + lo*hi by
+//                       three v_mfma_f32_32x32x16_bf16 passes: an error bound 3 to 11 times
+//                       smaller.  For base sets outside the half operands' range, and for
+//                       the repeat of a call of which they left too many rows uncertified.
 //   merge   : per result row, merges the partial rows of its candidate splits,
 //             re-scores the best EXACTLY in the reference's fp32 summation order and
 //             certifies, from a proven bound on the pre-selection's error, that no
@@ -65,12 +72,16 @@ struct MergeItem {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 struct SelectParams {
-    const uint32_t *xs; // split base set: [N][dp] words, see ung_split_kernel
+    const uint32_t *xs; // pre-selection operands: [N][dp] words, the half base set (ung_half_kernel)
+                        // or the split base set (ung_split_kernel)
     const float *xn;
-    uint32_t dp;        // words per split row = d rounded up to a multiple of KC
+    uint32_t dp;        // words per operand row, whole chunks of KC words
+    float s2, inv_s2;   // squared scale of the operands (a power of two; 1 for the split set) and
+                        // its inverse: the kernel works in scaled distances, partial rows do not
     uint32_t k;
     const Job *jobs;
     const Item *items;
@@ -79,9 +90,6 @@ struct SelectParams {
     uint32_t *part_ids;
     float *part_dist;
     float *part_bound;
-    double eps_coef;  // (7d/4+112)*2^-24 : expansion-form error factor on (|q|+R)^2
-    double shrink;    // (d/8+8)*2^-24 : relative error of the reference summation
-    double rmax;      // max candidate norm (slightly inflated)
     uint32_t n_items; // items of this launch
     uint32_t *item_ctr; // next item to take (zeroed before the launch)
     uint32_t lp;      // entries per partial row (approximate top-Lp)
@@ -307,16 +315,16 @@ __device__ __forceinline__ void list_insert(float (&ld)[LT], uint32_t (&li)[LT],
     li[0] = c_hi ? ni : li[0];
 }
 
-// Error term of one query, computed once per row: ea = eps_coef * (|q| + R)^2 (|q| from
-// the cached |q|^2, rounded up), with
-//   |a - D| <= eps_coef * (|q| + R)^2   (norm cache, MFMA dot, epilogue roundings)
+// Error term of one query, computed once per row: ea = eps_coef * r^2 + eps_lin * r with
+// r = |q| + R (|q| from the cached |q|^2, rounded up), and
+//   |a - D| <= ea   (operand roundings, norm cache, MFMA dot, epilogue roundings)
 //   e >= D * (1 - shrink), e <= D * (1 + shrink)   (reference summation)
 // for the expansion-form MFMA value a, the exact squared distance D and the reference's
 // rounded value e.
-__device__ __forceinline__ double bound_ea(float qn, double eps_coef, double rmax)
+__device__ __forceinline__ double bound_ea(float qn, double eps_coef, double eps_lin, double rmax)
 {
     const double r = sqrt((double)fmaxf(qn, 0.0f) * (1.0 + 1e-6)) + rmax;
-    return eps_coef * r * r;
+    return eps_coef * r * r + eps_lin * r;
 }
 
 // Lower bound on the exact (reference-rounded) distance of any candidate whose
@@ -410,19 +418,14 @@ struct alignas(16) SelectSmem {
 };
 static_assert(BQ == BC, "the epilogue staging addresses assume square panels");
 
-// Register-query layout (dp = 128, two query columns per lane): a lane keeps the high
-// bf16 words of its query columns for all 8 k-blocks in registers for the whole item,
-// and the low words of the item's queries stay resident in LDS; per step only the
-// candidate chunk is loaded and staged.  LDS traffic per step and wave: 8 KB of
-// candidate operands + 4 KB of query low words + 4 KB of staging writes, against 16 +
-// 8 KB when both panels are restaged every step.
-constexpr int QR_NK = 4;              // chunks of 32 dimensions (dp = 128)
-constexpr int QLO_W = QR_NK * 16 + 4; // words per resident low-word query row (padded)
+// Register-query layout (half operand rows of 128 dimensions, two query columns per lane): a
+// lane keeps its query columns' operands of all 8 k-blocks in registers for the whole item;
+// per step only the candidate chunk is loaded and staged.
+constexpr int QR_NK = 2; // chunks of 64 dimensions
 struct alignas(16) SelectSmemQ {
     union {
         struct {
             float4 xs[2][BC][LDSW / 4];
-            float4 qlo[BQ][QLO_W / 4];
         } p;
         SelectRed r;
     } u;
@@ -511,7 +514,7 @@ __device__ __forceinline__ float start_rowids(Smem &sm, int slot, RowCursor &cur
         uint32_t g = NONE;
         if (v < v_end) {
             g = cursor_id(cur, P, jb, v);
-            nx = P.xn[g];
+            nx = P.xn[g] * P.s2;
         }
         sm.rowid[slot][tid] = g;
     }
@@ -706,11 +709,11 @@ constexpr int select_threads()
     return NB == 2 ? NTHREADS : 2 * NTHREADS;
 }
 
-template <int LT, int MODE, bool EXCL, int NB, bool QR>
+template <int LT, int MODE, bool EXCL, int NB, bool QR, bool HALF>
 __global__ __launch_bounds__(select_threads<NB>(), (LT <= 8 ? 2 : 1)) void ung_select_kernel(SelectParams P)
 {
     static_assert(NB == 1 || NB == 2, "one or two query columns per lane");
-    static_assert(!QR || (NB == 2 && LT == 8), "register-query layout: NB = 2, LT = 8");
+    static_assert(!QR || (NB == 2 && LT == 8 && HALF), "register-query layout: NB = 2, LT = 8, half operands");
     constexpr int NTH = select_threads<NB>();
     constexpr int WN = 4 / NB;         // query waves
     constexpr int QW = 32 * NB;        // query columns per wave
@@ -742,7 +745,7 @@ __global__ __launch_bounds__(select_threads<NB>(), (LT <= 8 ? 2 : 1)) void ung_s
     const uint32_t *__restrict__ XS = P.xs;
 
     if (tid < BQ)
-        sm.qn[tid] = (uint32_t)tid < qcnt ? P.xn[q0 + tid] : 0.0f;
+        sm.qn[tid] = (uint32_t)tid < qcnt ? P.xn[q0 + tid] * P.s2 : 0.0f;
     RowCursor cur;
     finish_rowids(sm, 0, start_rowids(sm, 0, cur, P, jb, it.v_begin, it.v_end, tid), tid);
 
@@ -789,27 +792,18 @@ __global__ __launch_bounds__(select_threads<NB>(), (LT <= 8 ? 2 : 1)) void ung_s
     const uint32_t qrow_step = (uint32_t)RSTEP * dp * 4u;
     const uint32_t qoff = ((uint32_t)lr0 * dp + (uint32_t)c4) * 4u;
 
-    // register-query layout: the high words of this lane's query columns (k-block kb:
-    // chunk kb/2, float4 column 2*(kb%2) + h of the chunk row) and the low words of all
-    // the item's queries (float4 column 4*chunk + c of row q) into LDS
-    [[maybe_unused]] bf16x8 bhr[2 * QR_NK][NB];
+    // register-query layout: this lane's query columns, one float4 per k-block of 16
+    // dimensions (k-block kb: words 8 kb + 4 h .. +3 of the row)
+    [[maybe_unused]] halfx8 bhr[4 * QR_NK][NB];
     if constexpr (QR) {
         // rows of the item's queries (row 0 of qres is query q0; zeros past its qcnt rows)
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
             const uint32_t row = (uint32_t)(wn * QW + 32 * nb + r);
 #pragma unroll
-            for (int kb = 0; kb < 2 * QR_NK; ++kb)
+            for (int kb = 0; kb < 4 * QR_NK; ++kb)
                 bhr[kb][nb] = __builtin_bit_cast(
-                    bf16x8, __builtin_amdgcn_raw_buffer_load_b128(
-                                qres, (row * dp + (uint32_t)((kb >> 1) * KC + (2 * (kb & 1) + h) * 4)) * 4u, 0, 0));
-        }
-#pragma unroll
-        for (int i = 0; i < BQ * QR_NK * 4 / NTH; ++i) {
-            const int idx = tid + NTH * i;
-            const int q = idx >> 4, f = idx & 15; // f = 4*chunk + float4 column of the low words
-            const uint32_t off = ((uint32_t)q * dp + (uint32_t)((f >> 2) * KC + 16 + (f & 3) * 4)) * 4u;
-            sm.u.p.qlo[q][f] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(qres, off, 0, 0));
+                    halfx8, __builtin_amdgcn_raw_buffer_load_b128(qres, (row * dp + (uint32_t)(8 * kb + 4 * h)) * 4u, 0, 0));
         }
     }
 
@@ -895,16 +889,43 @@ __global__ __launch_bounds__(select_threads<NB>(), (LT <= 8 ? 2 : 1)) void ung_s
                 load_chunk((kc + 1) * KC);
             }
         }
-        // The chunk's 32 dimensions as two k-blocks of 16; a panel row holds the bf16 high
-        // parts of the 32 dimensions (words 0..15) then the low parts (words 16..31).
-        // Lane half h feeds dimensions 16*kb + 8h .. +7 of block kb (8 bf16 = one float4),
-        // the same k order for the candidate (A) and query (B) operands.  Three passes per
-        // block: hi*hi, hi*lo, lo*hi (the dropped lo*lo term is within the error bound);
-        // pass-major order keeps four independent accumulators between dependent MFMAs.
+        // A panel row is one chunk of an operand row (32 words).  Lane half h feeds dimensions
+        // 16*kb + 8h .. +7 of k-block kb (8 values = one float4), the same k order for the
+        // candidate (A) and query (B) operands.
+        //   HALF:  64 dimensions, four k-blocks, one product each;
+        //   split: 32 dimensions, two k-blocks -- the bf16 high parts in words 0..15, the low
+        //          parts in words 16..31; three passes per block: hi*hi, hi*lo, lo*hi (the
+        //          dropped lo*lo term is within the error bound), pass-major, so that four
+        //          independent accumulators lie between dependent MFMAs.
         // A tile's first MFMA of each accumulator takes C = 0 (no zeroing instructions).
         auto mfma_chunk = [&](auto first_chunk) {
             constexpr bool FIRST = decltype(first_chunk)::value;
             const floatx16 zero = {};
+            if constexpr (HALF) {
+#pragma unroll
+                for (int kb = 0; kb < 4; ++kb) {
+                    const int ch = 2 * kb + h;
+                    halfx8 a[2], b[NB];
+#pragma unroll
+                    for (int mb = 0; mb < 2; ++mb)
+                        a[mb] = __builtin_bit_cast(halfx8, sm.u.p.xs[buf][wm * 64 + 32 * mb + r][ch]);
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb) {
+                        if constexpr (QR) {
+                            constexpr int KCI = decltype(kcv)::value;
+                            b[nb] = bhr[4 * KCI + kb][nb];
+                        } else {
+                            b[nb] = __builtin_bit_cast(halfx8, sm.u.p.qs[buf][wn * QW + 32 * nb + r][ch]);
+                        }
+                    }
+#pragma unroll
+                    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+                        for (int nb = 0; nb < NB; ++nb)
+                            acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                                a[mb], b[nb], (FIRST && kb == 0) ? zero : acc[mb][nb], 0, 0, 0);
+                }
+            } else {
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb) {
                 const int ch = 2 * kb + h; // float4 column of the high parts; +4: low parts
@@ -916,14 +937,8 @@ __global__ __launch_bounds__(select_threads<NB>(), (LT <= 8 ? 2 : 1)) void ung_s
                 }
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb) {
-                    if constexpr (QR) {
-                        constexpr int KCI = decltype(kcv)::value;
-                        bh[nb] = bhr[2 * KCI + kb][nb];
-                        bl[nb] = __builtin_bit_cast(bf16x8, sm.u.p.qlo[wn * QW + 32 * nb + r][4 * KCI + ch]);
-                    } else {
-                        bh[nb] = __builtin_bit_cast(bf16x8, sm.u.p.qs[buf][wn * QW + 32 * nb + r][ch]);
-                        bl[nb] = __builtin_bit_cast(bf16x8, sm.u.p.qs[buf][wn * QW + 32 * nb + r][ch + 4]);
-                    }
+                    bh[nb] = __builtin_bit_cast(bf16x8, sm.u.p.qs[buf][wn * QW + 32 * nb + r][ch]);
+                    bl[nb] = __builtin_bit_cast(bf16x8, sm.u.p.qs[buf][wn * QW + 32 * nb + r][ch + 4]);
                 }
                 const bool z = FIRST && kb == 0;
 #pragma unroll
@@ -941,6 +956,7 @@ __global__ __launch_bounds__(select_threads<NB>(), (LT <= 8 ? 2 : 1)) void ung_s
 #pragma unroll
                     for (int nb = 0; nb < NB; ++nb)
                         acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[mb], bh[nb], acc[mb][nb], 0, 0, 0);
+            }
             }
         };
         // the MFMA block at raised wave priority: the SIMD's other wave (in its epilogue's
@@ -1299,8 +1315,6 @@ __global__ __launch_bounds__(select_threads<NB>(), (LT <= 8 ? 2 : 1)) void ung_s
         for (uint32_t s = 0; s < total; s += QR_NK) {
             step(s, std::integral_constant<uint32_t, 0>{});
             step(s + 1, std::integral_constant<uint32_t, 1>{});
-            step(s + 2, std::integral_constant<uint32_t, 2>{});
-            step(s + 3, std::integral_constant<uint32_t, 3>{});
         }
     } else {
         for (uint32_t s = 0; s < total; ++s)
@@ -1360,7 +1374,7 @@ __global__ __launch_bounds__(select_threads<NB>(), (LT <= 8 ? 2 : 1)) void ung_s
                     break;
                 }
                 P.part_ids[prow * Lp + t] = bi;
-                P.part_dist[prow * Lp + t] = bd;
+                P.part_dist[prow * Lp + t] = bd * P.inv_s2;
                 if (bl >= 0)
                     ++hp[bl];
             }
@@ -1368,7 +1382,7 @@ __global__ __launch_bounds__(select_threads<NB>(), (LT <= 8 ? 2 : 1)) void ung_s
 #pragma unroll
             for (int l = 0; l < 4; ++l)
                 A = fminf(A, sm.u.r.alist[jl][l]);
-            P.part_bound[prow] = A; // approximate-distance space
+            P.part_bound[prow] = A * P.inv_s2; // approximate-distance space
         }
     }
 }
@@ -1412,7 +1426,7 @@ constexpr uint32_t KNN_KEEP = 80;         // most entries a refresh keeps
 constexpr uint32_t KNN_OUT = 64;          // most entries the final refresh keeps (4 threads x 16)
 constexpr int KNN_THREADS = 512;          // 8 waves: 2 (candidate halves) x 4 (query quarters)
 constexpr uint32_t KNN_MAX_SPLIT = 65535; // candidates per item (16-bit candidate index)
-constexpr int KNN_MAX_NK = 4;             // dp <= 128
+constexpr uint32_t KNN_MAX_D = 128;       // the query column fits the lane's registers
 
 struct alignas(16) KnnSmem {
     float4 xs[2][BC][LDSW / 4];     // candidate chunks, double-buffered
@@ -1476,7 +1490,7 @@ __device__ __forceinline__ uint32_t quad_incl(uint32_t v, int p)
     return v + (p >= 2 ? b : 0u);
 }
 
-template <int MODE, int NK>
+template <int MODE, int NK, bool HALF>
 __global__ __launch_bounds__(KNN_THREADS, 1) void ung_knn_select_kernel(SelectParams P)
 {
     constexpr int NTH = KNN_THREADS;
@@ -1502,7 +1516,7 @@ __global__ __launch_bounds__(KNN_THREADS, 1) void ung_knn_select_kernel(SelectPa
     const uint32_t *__restrict__ XS = P.xs;
 
     if (tid < BQ) {
-        sm.qn[tid] = (uint32_t)tid < qcnt ? P.xn[q0 + tid] : 0.0f;
+        sm.qn[tid] = (uint32_t)tid < qcnt ? P.xn[q0 + tid] * P.s2 : 0.0f;
         sm.tau[tid] = INFINITY;
         sm.lost[tid] = ord_key(INFINITY);
         sm.fill[tid] = 0u;
@@ -1524,17 +1538,20 @@ __global__ __launch_bounds__(KNN_THREADS, 1) void ung_knn_select_kernel(SelectPa
         xres = __builtin_amdgcn_make_buffer_rsrc((void *)XS, (short)0, (int)P.x_bytes, 0x00020000);
     qres = __builtin_amdgcn_make_buffer_rsrc((void *)(XS + (size_t)q0 * DP), (short)0, (int)(qcnt * DP * 4u),
                                              0x00020000);
-    // this lane's query column for the whole item: the high and low words of every
-    // k-block (chunk kc, block kb: float4 column 2*kb + h of the chunk row, +4 for the
-    // low words); columns past the item's queries load zeros
-    bf16x8 qh[NK][2], ql[NK][2];
+    // this lane's query column for the whole item (columns past the item's queries load
+    // zeros).  HALF: k-block kb of chunk kc in float4 column 2*kb + h of the chunk row;
+    // split: its high words there, its low words in float4 column 2*kb + h + 4
+    constexpr int NKB = HALF ? 4 : 2; // k-blocks of 16 dimensions per chunk
+    u32x4 qh[NK][NKB];
+    [[maybe_unused]] u32x4 ql[NK][2];
 #pragma unroll
     for (int kc = 0; kc < NK; ++kc)
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
+        for (int kb = 0; kb < NKB; ++kb) {
             const uint32_t off = ((uint32_t)col * DP + (uint32_t)(kc * KC + (2 * kb + h) * 4)) * 4u;
-            qh[kc][kb] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(qres, off, 0, 0));
-            ql[kc][kb] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(qres, off + 64u, 0, 0));
+            qh[kc][kb] = __builtin_amdgcn_raw_buffer_load_b128(qres, off, 0, 0);
+            if constexpr (!HALF)
+                ql[kc][kb] = __builtin_amdgcn_raw_buffer_load_b128(qres, off + 64u, 0, 0);
         }
     auto set_xrows = [&](int slot) {
 #pragma unroll
@@ -1787,29 +1804,39 @@ __global__ __launch_bounds__(KNN_THREADS, 1) void ung_knn_select_kernel(SelectPa
                 set_xrows(next_slot);
                 load_chunk(0);
             }
-            // three bf16 passes per 16-dimension block (hi*hi, hi*lo, lo*hi); the tile's
-            // first MFMA of each accumulator takes C = 0
+            // HALF: one product per 16-dimension block; split: three bf16 passes (hi*hi,
+            // hi*lo, lo*hi); the tile's first MFMA of each accumulator takes C = 0
             __builtin_amdgcn_s_setprio(1);
             const floatx16 zero = {};
 #pragma unroll
-            for (int kb = 0; kb < 2; ++kb) {
+            for (int kb = 0; kb < NKB; ++kb) {
                 const int ch = 2 * kb + h;
-                bf16x8 ah[2], al[2];
+                const bool z = kc == 0 && kb == 0;
+                if constexpr (HALF) {
 #pragma unroll
-                for (int mb = 0; mb < 2; ++mb) {
-                    ah[mb] = __builtin_bit_cast(bf16x8, sm.xs[buf][wm * 64 + 32 * mb + r][ch]);
-                    al[mb] = __builtin_bit_cast(bf16x8, sm.xs[buf][wm * 64 + 32 * mb + r][ch + 4]);
+                    for (int mb = 0; mb < 2; ++mb)
+                        acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                            __builtin_bit_cast(halfx8, sm.xs[buf][wm * 64 + 32 * mb + r][ch]),
+                            __builtin_bit_cast(halfx8, qh[kc][kb]), z ? zero : acc[mb], 0, 0, 0);
+                } else {
+                    const bf16x8 bh = __builtin_bit_cast(bf16x8, qh[kc][kb]);
+                    const bf16x8 bl = __builtin_bit_cast(bf16x8, ql[kc][kb]);
+                    bf16x8 ah[2], al[2];
+#pragma unroll
+                    for (int mb = 0; mb < 2; ++mb) {
+                        ah[mb] = __builtin_bit_cast(bf16x8, sm.xs[buf][wm * 64 + 32 * mb + r][ch]);
+                        al[mb] = __builtin_bit_cast(bf16x8, sm.xs[buf][wm * 64 + 32 * mb + r][ch + 4]);
+                    }
+#pragma unroll
+                    for (int mb = 0; mb < 2; ++mb)
+                        acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[mb], bh, z ? zero : acc[mb], 0, 0, 0);
+#pragma unroll
+                    for (int mb = 0; mb < 2; ++mb)
+                        acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[mb], bl, acc[mb], 0, 0, 0);
+#pragma unroll
+                    for (int mb = 0; mb < 2; ++mb)
+                        acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[mb], bh, acc[mb], 0, 0, 0);
                 }
-#pragma unroll
-                for (int mb = 0; mb < 2; ++mb)
-                    acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[mb], qh[kc][kb],
-                                                                      (kc == 0 && kb == 0) ? zero : acc[mb], 0, 0, 0);
-#pragma unroll
-                for (int mb = 0; mb < 2; ++mb)
-                    acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[mb], ql[kc][kb], acc[mb], 0, 0, 0);
-#pragma unroll
-                for (int mb = 0; mb < 2; ++mb)
-                    acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[mb], qh[kc][kb], acc[mb], 0, 0, 0);
             }
             __builtin_amdgcn_s_setprio(0);
             if (NK > 1 && kc == 0 && more)
@@ -1964,11 +1991,11 @@ __global__ __launch_bounds__(KNN_THREADS, 1) void ung_knn_select_kernel(SelectPa
                 const uint32_t e = (uint32_t)(16 * p + i);
                 if (e < Lp) {
                     P.part_ids[prow * Lp + e] = d[i] < INFINITY ? id0 + id[i] : NONE;
-                    P.part_dist[prow * Lp + e] = d[i];
+                    P.part_dist[prow * Lp + e] = d[i] * P.inv_s2;
                 }
             }
             if (p == 0)
-                P.part_bound[prow] = fminf(sm.tau[q], next);
+                P.part_bound[prow] = fminf(sm.tau[q], next) * P.inv_s2;
         }
     }
 }
@@ -1987,7 +2014,7 @@ struct MergeParams {
     const float *part_bound;
     uint32_t lp;
     uint32_t k;
-    double eps_coef, shrink, rmax;
+    double eps_coef, eps_lin, shrink, rmax;
     uint32_t *out_ids;
     float *out_dist;
     int32_t *out_size;
@@ -2193,7 +2220,7 @@ __global__ __launch_bounds__(64 * MERGE_ROWS) void ung_merge_kernel(MergeParams 
     // exact distance > T (it is neither a result nor needed by the certificate).  The
     // candidates are in ascending approximate order, so the re-scored ones are a prefix.
     const float xq = M.xn[q];
-    const double ea = bound_ea(xq, M.eps_coef, M.rmax);
+    const double ea = bound_ea(xq, M.eps_coef, M.eps_lin, M.rmax);
     uint32_t m_need = Lp;
     if (k <= Lp) {
         const int src = (int)((k - 1u) & 63u);
@@ -2645,21 +2672,25 @@ __global__ __launch_bounds__(256) void ung_split_kernel(const float *__restrict_
     }
 }
 
-// Squared norms (one wave per row, grid-stride over rows; lanes stride the row) and the
-// largest of them: a block-wide maximum, then one atomic per block.  Accumulated in fp64
-// and rounded once, so each cached norm is within 2^-24 (relative) of |x|^2.
+// Squared norms (one wave per row, grid-stride over rows; lanes stride the row), the
+// largest of them (maxbits[0]) and the largest |coordinate| (maxbits[1]): block-wide maxima,
+// then one atomic per block.  Accumulated in fp64 and rounded once, so each cached norm is
+// within 2^-24 (relative) of |x|^2.  Non-negative floats order as their bit patterns (a NaN
+// or infinite coordinate gives an exponent of 255).
 __global__ __launch_bounds__(256) void ung_norm_kernel(const float *__restrict__ X, uint64_t N, uint32_t d,
                                                        float *__restrict__ xn, unsigned int *__restrict__ maxbits)
 {
-    __shared__ unsigned int wmax[4];
+    __shared__ unsigned int wmax[2][4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint64_t nwaves = (uint64_t)gridDim.x * 4u;
-    unsigned int mx = 0u; // non-negative floats order as their bit patterns
+    unsigned int mx = 0u, am = 0u;
     for (uint64_t row = (uint64_t)blockIdx.x * 4u + (uint64_t)wave; row < N; row += nwaves) {
         const float *x = X + row * d;
         double sd = 0.0;
-        for (uint32_t t = lane; t < d; t += 64)
+        for (uint32_t t = lane; t < d; t += 64) {
             sd = __builtin_fma((double)x[t], (double)x[t], sd);
+            am = max(am, __float_as_uint(x[t]) & 0x7FFFFFFFu);
+        }
         for (int off = 32; off > 0; off >>= 1)
             sd += __shfl_xor(sd, off);
         const float s = (float)sd;
@@ -2667,11 +2698,68 @@ __global__ __launch_bounds__(256) void ung_norm_kernel(const float *__restrict__
             xn[row] = s;
         mx = max(mx, __float_as_uint(s));
     }
+    for (int off = 32; off > 0; off >>= 1)
+        am = max(am, (unsigned int)__shfl_xor((int)am, off));
+    if (lane == 0) {
+        wmax[0][wave] = mx;
+        wmax[1][wave] = am;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2)
+        atomicMax(maxbits + threadIdx.x, max(max(wmax[threadIdx.x][0], wmax[threadIdx.x][1]),
+                                             max(wmax[threadIdx.x][2], wmax[threadIdx.x][3])));
+}
+
+// Power of two that takes the largest |coordinate| (exponent field e of its bits) into
+// [2^14, 2^15), below the fp16 maximum of 65504.  Only for e in [HALF_EMIN, HALF_EMAX]
+// (coordinates from 2^-40 to 2^40): beyond, scaled squared distances could leave the fp32
+// range, and the split operands are used.
+constexpr uint32_t HALF_EMIN = 127u - 40u, HALF_EMAX = 127u + 40u;
+__host__ __device__ inline uint32_t half_scale_bits(uint32_t e) { return (127u + 14u + 127u - e) << 23; }
+
+// The half base set: row n holds the d coordinates times the scale, rounded to fp16
+// (nearest even; below the fp16 normal range: 0), zeros up to hp words.  maxbits[2] gets
+// the largest squared norm (fp64 rounded up to fp32) of what the rounding left out of a
+// row, in the coordinates' own scale: the certificate's error term.  One wave per row.
+__global__ __launch_bounds__(256) void ung_half_kernel(const float *__restrict__ X, uint64_t N, uint32_t d,
+                                                       uint32_t hp, uint32_t *__restrict__ XH,
+                                                       unsigned int *__restrict__ maxbits)
+{
+    __shared__ unsigned int wmax[4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t e = maxbits[1] >> 23;
+    if (e < HALF_EMIN || e > HALF_EMAX)
+        return; // (the host applies the same rule and does not use XH)
+    const float scale = __uint_as_float(half_scale_bits(e));
+    const float inv = 1.0f / scale; // exact
+    const uint64_t nwaves = (uint64_t)gridDim.x * 4u;
+    unsigned int mx = 0u;
+    for (uint64_t row = (uint64_t)blockIdx.x * 4u + (uint64_t)wave; row < N; row += nwaves) {
+        const float *x = X + row * d;
+        double rd = 0.0;
+        for (uint32_t w = (uint32_t)lane; w < hp; w += 64u) {
+            uint32_t bits = 0u;
+#pragma unroll
+            for (uint32_t j = 0; j < 2; ++j) {
+                const uint32_t dim = 2u * w + j;
+                const float v = dim < d ? x[dim] : 0.0f;
+                const float sv = v * scale;
+                const _Float16 hv = fabsf(sv) < 0x1p-14f ? (_Float16)0.0f : (_Float16)sv;
+                const float rv = v - (float)hv * inv; // exact
+                rd = __builtin_fma((double)rv, (double)rv, rd);
+                bits |= (uint32_t)__builtin_bit_cast(uint16_t, hv) << (16u * j);
+            }
+            XH[row * hp + w] = bits;
+        }
+        for (int off = 32; off > 0; off >>= 1)
+            rd += __shfl_xor(rd, off);
+        mx = max(mx, __float_as_uint(__double2float_ru(rd)));
+    }
     if (lane == 0)
         wmax[wave] = mx;
     __syncthreads();
     if (threadIdx.x == 0)
-        atomicMax(maxbits, max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3])));
+        atomicMax(maxbits + 2, max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3])));
 }
 
 __global__ void ung_fill_rows_kernel(uint32_t *ids, float *dist, int32_t *size, uint64_t rows,

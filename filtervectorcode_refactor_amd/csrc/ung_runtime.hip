@@ -146,6 +146,7 @@ struct Plan {
     // entries per partial row of the cross call whose partial rows are still in the
     // first workspace (set when such a call succeeds; 0: none)
     uint32_t part_lp = 0;
+    bool part_half = false; // their operands (PlanMem::half)
 };
 
 
@@ -216,6 +217,10 @@ struct PlanMem {
     int32_t *out_size = nullptr;
     std::vector<uint32_t> *rescanned = nullptr; // output rows that took the exact rescan
     char *stage = nullptr;          // host staging (stage_layout), stable until the call ends
+    // pre-selection of the call: half operands (one fp16 product) or split ones (three bf16
+    // products), and its entries per partial row
+    bool half = false;
+    uint32_t lp = 0;
     // rescan range partials: grown in the workspace on demand, or a fixed region
     bool fb_grow = true;
     uint32_t *fb_ids = nullptr;
@@ -272,6 +277,11 @@ struct ung_hip_ctx {
     float *X = nullptr;
     uint32_t *XS = nullptr; // split base set (bf16 hi/lo pairs) for the MFMA pre-selection
     uint32_t dp = 0;        // its row pitch in words
+    uint32_t *XH = nullptr; // half base set (scaled fp16) for the MFMA pre-selection
+    uint32_t hp = 0;        // its row pitch in words
+    bool half_ok = false;   // XH is usable (half_rule)
+    float half_s2 = 1.0f;   // its squared scale
+    double half_res = 0.0;  // largest norm of what the fp16 rounding left out of a row (rounded up)
     float *xn = nullptr;
     unsigned int *maxbits = nullptr;
     uint64_t N = 0;
@@ -331,6 +341,8 @@ struct ung_hip_ctx {
     // test hook: UNG_HIP_NO_QREG=1 at create keeps the select kernel's restaged query panel
     // where the register-query layout would apply
     bool qreg = true;
+    // test hook: UNG_HIP_NO_HALF=1 at create keeps every pre-selection on the split operands
+    bool half = true;
     // test hook: UNG_HIP_EPS_SCALE=s (s >= 1) at create widens the certification error
     // bound by s, which sends more rows (all, for a huge s) through the exact rescan
     double eps_scale = 1.0;
@@ -424,14 +436,20 @@ void add_pack_items(Plan &pl)
     }
 }
 
-// Entries per partial row: the k results plus a margin, at most two per merge lane
-// and at most the 4 queues' entries.  The certified error bound grows with d; from
-// d = 512 a margin of 10 keeps the first value left out far enough above the k-th
-// that few rows need the exact rescan (cfg4: 133 rescanned cross rows, 4.5 ms, with a
-// margin of 4), while at d = 128 the longer rows cost more than the rescans they save.
-uint32_t pick_lp(uint32_t k, int lt, uint32_t d)
+// Entries per partial row past the k results.  The certified error bound grows with d, and
+// the half operands' is the wider one; a margin of 10 keeps the first value left out far
+// enough above the k-th that few rows need the exact rescan (cfg4, split operands: 133
+// rescanned cross rows, 4.5 ms, with a margin of 4; cfg2, half operands: about one row in
+// 750 with a margin of 4, none in 1,500 with 6), while with the split operands at d = 128
+// the longer rows cost more than the rescans they save.
+uint32_t lp_margin(uint32_t k, uint32_t d, bool half)
 {
-    const uint32_t margin = std::max<uint32_t>(d >= 512u ? 10u : 4u, k / 4);
+    return std::max<uint32_t>(half || d >= 512u ? 10u : 4u, k / 4);
+}
+
+// Entries per partial row: at most two per merge lane and at most the 4 queues' entries.
+uint32_t pick_lp(uint32_t k, int lt, uint32_t margin)
+{
     return std::min<uint32_t>(std::min<uint32_t>(128u, 4u * (uint32_t)lt), k + margin);
 }
 
@@ -445,99 +463,110 @@ int pick_lt(uint32_t k)
     return 32;
 }
 
-template <int LT>
-int launch_select_t(ung_hip_ctx *ctx, hipStream_t stream, const SelectParams &P, uint32_t n_items, bool excl)
+// Operands of a pre-selection and the constants of its certified error bound
+// |a - D| <= coef * r^2 + lin * r, r = |q| + rmax (bound_ea).
+struct Operands {
+    const uint32_t *xs = nullptr;
+    uint32_t dp = 0; // row pitch in words
+    float s2 = 1.0f;
+    double coef = 0.0, lin = 0.0, rmax = 0.0;
+};
+Operands operands_of(const ung_hip_ctx *ctx, bool half);
+
+// Load mode of an operand set: 32-bit buffer offsets below 4 GiB.
+int load_mode(const ung_hip_ctx *ctx, uint32_t dp)
 {
-    // 32-bit buffer offsets need a split base set below 4 GiB
-    const uint64_t x_bytes = (uint64_t)ctx->N * ctx->dp * sizeof(uint32_t);
-    const int mode = (x_bytes < (1ull << 32) && !ctx->force_wide) ? LOAD_BUF32 : LOAD_WIDE;
-    // grid dimension x is limited to 2^31-1; chunk the item list
+    return (uint64_t)ctx->N * dp * sizeof(uint32_t) < (1ull << 32) && !ctx->force_wide ? LOAD_BUF32 : LOAD_WIDE;
+}
+
+// Launches `kernel` over the items of P, chunked to the limit of grid dimension x.
+template <class K>
+int launch_items(ung_hip_ctx *ctx, hipStream_t stream, const SelectParams &P, uint32_t n_items, int mode, int threads,
+                 K kernel)
+{
     const uint32_t max_grid = 1u << 30;
     for (uint32_t off = 0; off < n_items; off += max_grid) {
         SelectParams Q = P;
         Q.items = P.items + off;
-        Q.x_bytes = mode == LOAD_BUF32 ? (uint32_t)x_bytes : 0u;
-        const uint32_t n = std::min(max_grid, n_items - off);
-        Q.n_items = n;
+        Q.x_bytes = mode == LOAD_BUF32 ? (uint32_t)(ctx->N * P.dp * sizeof(uint32_t)) : 0u;
+        Q.n_items = std::min(max_grid, n_items - off);
         if (off > 0) { // the counter was zeroed for the first chunk by the caller
             hipLaunchKernelGGL(ung_zero_u32_kernel, dim3(1), dim3(64), 0, stream, P.item_ctr, 1u);
             HIPCHECK(hipGetLastError());
         }
-        // queues longer than 8 take the one-column-per-lane layout (two waves per SIMD)
-        constexpr int NB = LT <= 8 ? 2 : 1;
-        const dim3 g(n), b(select_threads<NB>());
-        // two columns per lane and dp = 128: the register-query layout
-        const bool qr = NB == 2 && ctx->dp == (uint32_t)(QR_NK * KC) && ctx->qreg;
-        if constexpr (NB == 2) {
-            if (qr && mode == LOAD_BUF32 && excl)
-                hipLaunchKernelGGL((ung_select_kernel<LT, LOAD_BUF32, true, NB, true>), g, b, 0, stream, Q);
-            else if (qr && mode == LOAD_BUF32)
-                hipLaunchKernelGGL((ung_select_kernel<LT, LOAD_BUF32, false, NB, true>), g, b, 0, stream, Q);
-            else if (qr && excl)
-                hipLaunchKernelGGL((ung_select_kernel<LT, LOAD_WIDE, true, NB, true>), g, b, 0, stream, Q);
-            else if (qr)
-                hipLaunchKernelGGL((ung_select_kernel<LT, LOAD_WIDE, false, NB, true>), g, b, 0, stream, Q);
-        }
-        if (qr)
-            ; // launched above
-        else if (mode == LOAD_BUF32 && excl)
-            hipLaunchKernelGGL((ung_select_kernel<LT, LOAD_BUF32, true, NB, false>), g, b, 0, stream, Q);
-        else if (mode == LOAD_BUF32)
-            hipLaunchKernelGGL((ung_select_kernel<LT, LOAD_BUF32, false, NB, false>), g, b, 0, stream, Q);
-        else if (excl)
-            hipLaunchKernelGGL((ung_select_kernel<LT, LOAD_WIDE, true, NB, false>), g, b, 0, stream, Q);
-        else
-            hipLaunchKernelGGL((ung_select_kernel<LT, LOAD_WIDE, false, NB, false>), g, b, 0, stream, Q);
+        hipLaunchKernelGGL(kernel, dim3(Q.n_items), dim3(threads), 0, stream, Q);
         HIPCHECK(hipGetLastError());
     }
     return UNG_HIP_OK;
 }
 
-// Filter-and-buffer select of a group plan (ung_knn_select_kernel, dp <= 128), grid
-// chunked like launch_select_t.
-template <int NK>
+template <int LT, bool HALF>
+int launch_select_t(ung_hip_ctx *ctx, hipStream_t stream, const SelectParams &P, uint32_t n_items, bool excl)
+{
+    const int mode = load_mode(ctx, P.dp);
+    // queues longer than 8 take the one-column-per-lane layout (two waves per SIMD)
+    constexpr int NB = LT <= 8 ? 2 : 1;
+    const int th = select_threads<NB>();
+    if constexpr (NB == 2 && HALF) {
+        // two columns per lane and half operands of 128 dimensions: the register-query layout
+        if (P.dp == (uint32_t)(QR_NK * KC) && ctx->qreg) {
+            if (mode == LOAD_BUF32)
+                return excl ? launch_items(ctx, stream, P, n_items, mode, th, ung_select_kernel<LT, LOAD_BUF32, true, NB, true, HALF>)
+                            : launch_items(ctx, stream, P, n_items, mode, th, ung_select_kernel<LT, LOAD_BUF32, false, NB, true, HALF>);
+            return excl ? launch_items(ctx, stream, P, n_items, mode, th, ung_select_kernel<LT, LOAD_WIDE, true, NB, true, HALF>)
+                        : launch_items(ctx, stream, P, n_items, mode, th, ung_select_kernel<LT, LOAD_WIDE, false, NB, true, HALF>);
+        }
+    }
+    if (mode == LOAD_BUF32)
+        return excl ? launch_items(ctx, stream, P, n_items, mode, th, ung_select_kernel<LT, LOAD_BUF32, true, NB, false, HALF>)
+                    : launch_items(ctx, stream, P, n_items, mode, th, ung_select_kernel<LT, LOAD_BUF32, false, NB, false, HALF>);
+    return excl ? launch_items(ctx, stream, P, n_items, mode, th, ung_select_kernel<LT, LOAD_WIDE, true, NB, false, HALF>)
+                : launch_items(ctx, stream, P, n_items, mode, th, ung_select_kernel<LT, LOAD_WIDE, false, NB, false, HALF>);
+}
+
+template <bool HALF>
+int launch_select(ung_hip_ctx *ctx, hipStream_t stream, const SelectParams &P, uint32_t n_items, bool excl, int lt)
+{
+    if (lt == 8)
+        return launch_select_t<8, HALF>(ctx, stream, P, n_items, excl);
+    if (lt == 16)
+        return launch_select_t<16, HALF>(ctx, stream, P, n_items, excl);
+    return launch_select_t<32, HALF>(ctx, stream, P, n_items, excl);
+}
+
+// Filter-and-buffer select of a group plan (ung_knn_select_kernel, d <= 128).
+template <int NK, bool HALF>
 int launch_knn_select_t(ung_hip_ctx *ctx, hipStream_t stream, const SelectParams &P, uint32_t n_items)
 {
-    const uint64_t x_bytes = (uint64_t)ctx->N * ctx->dp * sizeof(uint32_t);
-    const int mode = (x_bytes < (1ull << 32) && !ctx->force_wide) ? LOAD_BUF32 : LOAD_WIDE;
-    const uint32_t max_grid = 1u << 30;
-    for (uint32_t off = 0; off < n_items; off += max_grid) {
-        SelectParams Q = P;
-        Q.items = P.items + off;
-        Q.x_bytes = mode == LOAD_BUF32 ? (uint32_t)x_bytes : 0u;
-        const uint32_t n = std::min(max_grid, n_items - off);
-        Q.n_items = n;
-        if (off > 0) {
-            hipLaunchKernelGGL(ung_zero_u32_kernel, dim3(1), dim3(64), 0, stream, P.item_ctr, 1u);
-            HIPCHECK(hipGetLastError());
-        }
-        if (mode == LOAD_BUF32)
-            hipLaunchKernelGGL((ung_knn_select_kernel<LOAD_BUF32, NK>), dim3(n), dim3(KNN_THREADS), 0, stream, Q);
-        else
-            hipLaunchKernelGGL((ung_knn_select_kernel<LOAD_WIDE, NK>), dim3(n), dim3(KNN_THREADS), 0, stream, Q);
-        HIPCHECK(hipGetLastError());
-    }
-    return UNG_HIP_OK;
+    const int mode = load_mode(ctx, P.dp);
+    return mode == LOAD_BUF32
+               ? launch_items(ctx, stream, P, n_items, mode, KNN_THREADS, ung_knn_select_kernel<LOAD_BUF32, NK, HALF>)
+               : launch_items(ctx, stream, P, n_items, mode, KNN_THREADS, ung_knn_select_kernel<LOAD_WIDE, NK, HALF>);
 }
 
-int launch_knn_select(ung_hip_ctx *ctx, hipStream_t stream, const SelectParams &P, uint32_t n_items)
+int launch_knn_select(ung_hip_ctx *ctx, hipStream_t stream, const SelectParams &P, uint32_t n_items, bool half)
 {
-    switch (ctx->dp / KC) {
+    switch (P.dp / KC * (half ? 10u : 1u)) {
+    case 10:
+        return launch_knn_select_t<1, true>(ctx, stream, P, n_items);
+    case 20:
+        return launch_knn_select_t<2, true>(ctx, stream, P, n_items);
     case 1:
-        return launch_knn_select_t<1>(ctx, stream, P, n_items);
+        return launch_knn_select_t<1, false>(ctx, stream, P, n_items);
     case 2:
-        return launch_knn_select_t<2>(ctx, stream, P, n_items);
+        return launch_knn_select_t<2, false>(ctx, stream, P, n_items);
     case 3:
-        return launch_knn_select_t<3>(ctx, stream, P, n_items);
+        return launch_knn_select_t<3, false>(ctx, stream, P, n_items);
     case 4:
-        return launch_knn_select_t<4>(ctx, stream, P, n_items);
+        return launch_knn_select_t<4, false>(ctx, stream, P, n_items);
     default:
-        set_error("filter-and-buffer select: dp=%u above %d", ctx->dp, KNN_MAX_NK * KC);
+        set_error("filter-and-buffer select: operand rows of %u words", P.dp);
         return UNG_HIP_EINVAL;
     }
 }
 
-// Error factor of the expansion-form value a = fl(|q|^2 - 2*acc) of the select kernel:
+// Error factor of the expansion-form value a = fl(|q|^2 - 2*acc) of the select kernel on the
+// split operands:
 // |a - D| <= eps_coef * (|q| + R)^2 with D the exact squared distance, u = 2^-24.
 //  * norm caches fl(|x|^2), fl(|q|^2): fp64 sums rounded once, <= u relative each
 //                                                                     -> u (|q|+R)^2
@@ -563,11 +592,54 @@ double eps_coef_for(uint32_t d)
     return (1.75 * (double)d + 132.0) * std::ldexp(1.0, -24);
 }
 
+// The same for the half operands, h(x) = x - res(x) with |res(x)| <= rho over the base set
+// (measured when the set is prepared), r = |q| + R + rho:
+//  * <x,q> - <h(x),h(q)> = <res(x),q> + <h(x),res(q)>, at most rho (|q| + |x| + rho) in s, so
+//    <= 2 rho r in a: the linear term;
+//  * the products of two 11-bit significands are exact in fp32; their accumulation over
+//    hp/16 MFMAs, in the fused-adder model above: 17/16 n u |h(x)||h(q)| with n = 2 hp
+//    dimensions, in a <= 0.54 n u r^2;
+//  * norm caches, norm term, bound and final fma as above: 21.1 u r^2 (the power-of-two
+//    scale changes no rounding).
+double eps_half_for(uint32_t hp) { return (0.6 * 2.0 * (double)hp + 32.0) * std::ldexp(1.0, -24); }
+
+Operands operands_of(const ung_hip_ctx *ctx, bool half)
+{
+    Operands o;
+    if (half) {
+        o.xs = ctx->XH;
+        o.dp = ctx->hp;
+        o.s2 = ctx->half_s2;
+        o.coef = eps_half_for(ctx->hp) * ctx->eps_scale;
+        o.lin = 2.0 * ctx->half_res * ctx->eps_scale;
+        o.rmax = ctx->rmax + ctx->half_res;
+    } else {
+        o.xs = ctx->XS;
+        o.dp = ctx->dp;
+        o.coef = eps_coef_for(ctx->d) * ctx->eps_scale;
+        o.rmax = ctx->rmax;
+    }
+    return o;
+}
+
+// Operands and partial-row length of a call.  Group lists keep the margin of the split
+// operands and take the half ones where it is at least 8 (k >= 32, or d >= 512): on 1,500
+// to 3,000 rows of cfg2, cfg3 and cfg4 none of their 32nd neighbours is within the half
+// operands' error bound of the 41st.
+void pick_operands(const ung_hip_ctx *ctx, uint32_t k, bool group, bool half, PlanMem &m)
+{
+    const uint32_t split_margin = lp_margin(k, ctx->d, false);
+    m.half = half && ctx->half_ok && (!group || split_margin >= 8u);
+    m.lp = pick_lp(k, pick_lt(k), m.half && !group ? lp_margin(k, ctx->d, true) : split_margin);
+}
+
 // PlanMem in the workspace's own buffers, grown to the plan (hipMalloc / hipHostMalloc
 // when a buffer is too small); rows into `res`.
-int workspace_mem(Workspace &ws, const Plan &pl, uint32_t lp, ResultBufs &res, PlanMem &m)
+int workspace_mem(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, ResultBufs &res, PlanMem &m)
 {
     int rc;
+    pick_operands(ctx, k, !pl.jobs.empty() && (pl.jobs[0].flags & 1u) != 0, true, m);
+    const uint32_t lp = m.lp;
     if ((rc = ws.jobs.ensure(pl.jobs.size())) || (rc = ws.items.ensure(pl.items.size())) ||
         (rc = ws.mitems.ensure(pl.n_mitems)) || (rc = ws.seg_start.ensure(pl.seg_start.size())) ||
         (rc = ws.seg_vend.ensure(pl.seg_vend.size())) ||
@@ -688,14 +760,14 @@ size_t merge_qlds_bytes(uint32_t d)
 // plan_launch uploads the work lists and enqueues the select and merge kernels;
 // plan_finish reads the flagged-row count back, rescans those rows and collects the
 // statistics.
-int plan_launch_merge(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, PlanMem &m, ung_hip_stats *st);
+int plan_launch_select(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, PlanMem &m);
+int plan_launch_merge(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, PlanMem &m, ung_hip_stats *st,
+                      bool upload);
 
 int plan_launch(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, PlanMem &m, ung_hip_stats *st,
                 hipEvent_t start_after = nullptr)
 {
     int rc;
-    const int lt = pick_lt(k);
-    const uint32_t lp = pick_lp(k, lt, ctx->d);
     const auto t_h2d = clk::now();
     const StageLayout L = stage_layout(pl);
     char *hs = m.stage;
@@ -716,44 +788,8 @@ int plan_launch(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, Pla
     // kernels of this plan start after `start_after` (another stream's event), if given
     if (start_after)
         HIPCHECK(hipStreamWaitEvent(ws.stream, start_after, 0));
-    hipLaunchKernelGGL(ung_zero_u32_kernel, dim3(1), dim3(64), 0, ws.stream, m.flag_count, 2u);
-    HIPCHECK(hipGetLastError());
-    HIPCHECK(hipEventRecord(ws.ev[0], ws.stream));
-
-    SelectParams P{};
-    P.xs = ctx->XS;
-    P.xn = ctx->xn;
-    P.dp = ctx->dp;
-    P.k = k;
-    P.jobs = m.jobs;
-    P.items = m.items;
-    P.seg_start = m.seg_start;
-    P.seg_vend = m.seg_vend;
-    P.part_ids = m.part_ids;
-    P.part_dist = m.part_dist;
-    P.part_bound = m.part_bound;
-    P.eps_coef = eps_coef_for(ctx->d) * ctx->eps_scale;
-    P.shrink = ((double)ctx->d / 8.0 + 8.0) * std::ldexp(1.0, -24);
-    P.rmax = ctx->rmax;
-    P.item_ctr = m.flag_count + 1;
-    P.lp = lp;
-    const uint32_t n_items = (uint32_t)pl.items.size();
-    const bool excl = (pl.jobs[0].flags & 1u) != 0; // one kind of job per plan
-    // group kNN lists with partial rows below 64 entries, splits below 65,536 candidates
-    // and d <= 128 (the mid-group batch of the exact kNN stage): the filter-and-buffer select
-    const bool knn = ctx->knn && excl && lp + 1u <= KNN_OUT && pl.max_item_cand <= KNN_MAX_SPLIT &&
-                     ctx->dp <= (uint32_t)(KNN_MAX_NK * KC);
-    if (knn)
-        rc = launch_knn_select(ctx, ws.stream, P, n_items);
-    else if (lt == 8)
-        rc = launch_select_t<8>(ctx, ws.stream, P, n_items, excl);
-    else if (lt == 16)
-        rc = launch_select_t<16>(ctx, ws.stream, P, n_items, excl);
-    else
-        rc = launch_select_t<32>(ctx, ws.stream, P, n_items, excl);
-    if (rc)
+    if ((rc = plan_launch_select(ctx, ws, pl, k, m)))
         return rc;
-    HIPCHECK(hipEventRecord(ws.ev[1], ws.stream));
     if (pl.n_tiny > 0) {
         // the jobs left out of the select (tiny_job), one wave each, exact
         FallbackParams F{};
@@ -774,26 +810,71 @@ int plan_launch(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, Pla
                            dim3(64 * TINY_WAVES), 0, ws.stream, F);
         HIPCHECK(hipGetLastError());
     }
-    return plan_launch_merge(ctx, ws, pl, k, m, st);
+    return plan_launch_merge(ctx, ws, pl, k, m, st, true);
 }
 
-// The merge of a launched plan, after its select kernel on ws.stream.
-int plan_launch_merge(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, PlanMem &m, ung_hip_stats *st)
+// The select of a plan whose work lists are on the device, on ws.stream (flags and item
+// counter cleared first).
+int plan_launch_select(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, PlanMem &m)
+{
+    int rc;
+    hipLaunchKernelGGL(ung_zero_u32_kernel, dim3(1), dim3(64), 0, ws.stream, m.flag_count, 2u);
+    HIPCHECK(hipGetLastError());
+    HIPCHECK(hipEventRecord(ws.ev[0], ws.stream));
+
+    const Operands o = operands_of(ctx, m.half);
+    const uint32_t lp = m.lp;
+    SelectParams P{};
+    P.xs = o.xs;
+    P.xn = ctx->xn;
+    P.dp = o.dp;
+    P.s2 = o.s2;
+    P.inv_s2 = 1.0f / o.s2;
+    P.k = k;
+    P.jobs = m.jobs;
+    P.items = m.items;
+    P.seg_start = m.seg_start;
+    P.seg_vend = m.seg_vend;
+    P.part_ids = m.part_ids;
+    P.part_dist = m.part_dist;
+    P.part_bound = m.part_bound;
+    P.item_ctr = m.flag_count + 1;
+    P.lp = lp;
+    const uint32_t n_items = (uint32_t)pl.items.size();
+    const bool excl = (pl.jobs[0].flags & 1u) != 0; // one kind of job per plan
+    // group kNN lists with partial rows below 64 entries, splits below 65,536 candidates
+    // and d <= 128 (the mid-group batch of the exact kNN stage): the filter-and-buffer select
+    const bool knn = ctx->knn && excl && lp + 1u <= KNN_OUT && pl.max_item_cand <= KNN_MAX_SPLIT && ctx->d <= KNN_MAX_D;
+    rc = knn      ? launch_knn_select(ctx, ws.stream, P, n_items, m.half)
+         : m.half ? launch_select<true>(ctx, ws.stream, P, n_items, excl, pick_lt(k))
+                  : launch_select<false>(ctx, ws.stream, P, n_items, excl, pick_lt(k));
+    if (rc)
+        return rc;
+    HIPCHECK(hipEventRecord(ws.ev[1], ws.stream));
+    return UNG_HIP_OK;
+}
+
+// The merge of a launched plan, after its select kernel on ws.stream; upload: its merge
+// items are not on the device yet.
+int plan_launch_merge(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, PlanMem &m, ung_hip_stats *st,
+                      bool upload)
 {
     if (pl.jobs.empty())
         return UNG_HIP_OK;
-    const uint32_t lp = pick_lp(k, pick_lt(k), ctx->d);
-    const StageLayout L = stage_layout(pl);
-    char *hs = m.stage;
-    // merge items, built and uploaded (on the upload stream) while the select kernel runs
-    const auto t_mi = clk::now();
-    write_merge_items(pl, reinterpret_cast<MergeItem *>(hs + L.om));
-    HIPCHECK(hipMemcpyAsync(m.mitems, hs + L.om, L.bm, hipMemcpyHostToDevice, ws.upload));
-    HIPCHECK(hipEventRecord(ws.ev_up, ws.upload));
-    HIPCHECK(hipStreamWaitEvent(ws.stream, ws.ev_up, 0));
+    if (upload) {
+        // built and uploaded (on the upload stream) while the select kernel runs
+        const StageLayout L = stage_layout(pl);
+        char *hs = m.stage;
+        const auto t_mi = clk::now();
+        write_merge_items(pl, reinterpret_cast<MergeItem *>(hs + L.om));
+        HIPCHECK(hipMemcpyAsync(m.mitems, hs + L.om, L.bm, hipMemcpyHostToDevice, ws.upload));
+        HIPCHECK(hipEventRecord(ws.ev_up, ws.upload));
+        HIPCHECK(hipStreamWaitEvent(ws.stream, ws.ev_up, 0));
+        if (st)
+            st->h2d_ms += ms_since(t_mi);
+    }
     HIPCHECK(hipEventRecord(ws.ev[4], ws.stream));
-    if (st)
-        st->h2d_ms += ms_since(t_mi);
+    const Operands o = operands_of(ctx, m.half);
 
     MergeParams M{};
     M.X = ctx->X;
@@ -804,11 +885,12 @@ int plan_launch_merge(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t 
     M.part_ids = m.part_ids;
     M.part_dist = m.part_dist;
     M.part_bound = m.part_bound;
-    M.lp = lp;
+    M.lp = m.lp;
     M.k = k;
-    M.eps_coef = eps_coef_for(ctx->d) * ctx->eps_scale;
+    M.eps_coef = o.coef;
+    M.eps_lin = o.lin;
     M.shrink = ((double)ctx->d / 8.0 + 8.0) * std::ldexp(1.0, -24);
-    M.rmax = ctx->rmax;
+    M.rmax = o.rmax;
     M.out_ids = m.out_ids;
     M.out_dist = m.out_dist;
     M.out_size = m.out_size;
@@ -849,6 +931,14 @@ int plan_launch_merge(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t 
 constexpr uint32_t FALLBACK_RANGE = 256;
 constexpr uint32_t MAX_FALLBACK_SPLITS = 1024;
 
+// A half pre-selection that leaves more than one row in HALF_RETRY uncertified (and more
+// than HALF_RETRY_MIN, below which the rescan takes less than another launch) is repeated on
+// the split operands before the rescan.  The exact rescan handles about 2.3e9 pairs/s at
+// d = 128 (cfg2: 14,060 rows of 27,400 candidates, 170 ms), the split select 1.4e12
+// (20.6e9 pairs, 14.4 ms): repeating pays from about one row in 600 on.
+constexpr uint32_t HALF_RETRY = 512;
+constexpr uint32_t HALF_RETRY_MIN = 256;
+
 int plan_finish(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, PlanMem &m, ung_hip_stats *st)
 {
     int rc;
@@ -857,6 +947,22 @@ int plan_finish(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, Pla
     uint32_t nflag = 0;
     HIPCHECK(hipMemcpyAsync(&nflag, m.flag_count, sizeof(uint32_t), hipMemcpyDeviceToHost, ws.stream));
     HIPCHECK(hipStreamSynchronize(ws.stream));
+    if (m.half && nflag > HALF_RETRY_MIN && (uint64_t)nflag * HALF_RETRY > pl.rows) {
+        if (st) {
+            float a = 0, b = 0;
+            HIPCHECK(hipEventElapsedTime(&a, ws.ev[0], ws.ev[1]));
+            HIPCHECK(hipEventElapsedTime(&b, ws.ev[4], ws.ev[2]));
+            st->select_ms += a;
+            st->merge_ms += b;
+            st->kernel_ms += a + b;
+            st->select_launches += 1;
+        }
+        pick_operands(ctx, k, (pl.jobs[0].flags & 1u) != 0, false, m); // (its partial rows are no longer than the half ones)
+        if ((rc = plan_launch_select(ctx, ws, pl, k, m)) || (rc = plan_launch_merge(ctx, ws, pl, k, m, st, false)))
+            return rc;
+        HIPCHECK(hipMemcpyAsync(&nflag, m.flag_count, sizeof(uint32_t), hipMemcpyDeviceToHost, ws.stream));
+        HIPCHECK(hipStreamSynchronize(ws.stream));
+    }
     if (nflag > 0) {
         // a flagged row's union is cut into ranges of >= FALLBACK_RANGE candidates
         uint64_t max_cand = 0;
@@ -926,7 +1032,7 @@ int plan_finish(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, Pla
         uint64_t rows_streamed = 0;
         for (const Item &it : pl.items)
             rows_streamed += (uint64_t)it.q_cnt + (it.v_end - it.v_begin);
-        st->select_bytes += rows_streamed * ctx->dp * sizeof(uint32_t);
+        st->select_bytes += rows_streamed * operands_of(ctx, m.half).dp * sizeof(uint32_t);
         st->rows += pl.rows;
         st->work_items += pl.items.size();
         st->select_launches += 1;
@@ -934,14 +1040,23 @@ int plan_finish(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, Pla
     return UNG_HIP_OK;
 }
 
+// The partial rows of a finished call on the first workspace, for the diagnostics.
+void keep_partials(Plan &pl, const PlanMem &m)
+{
+    pl.part_lp = m.lp;
+    pl.part_half = m.half;
+}
+
 // Launch + finish in the workspace's own (growable) memory, rows into `res`.
-int run_plan(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, ResultBufs &res, ung_hip_stats *st)
+int run_plan(ung_hip_ctx *ctx, Workspace &ws, Plan &pl, uint32_t k, ResultBufs &res, ung_hip_stats *st)
 {
     int rc;
     PlanMem m;
-    if ((rc = workspace_mem(ws, pl, pick_lp(k, pick_lt(k), ctx->d), res, m)) || (rc = plan_launch(ctx, ws, pl, k, m, st)))
+    if ((rc = workspace_mem(ctx, ws, pl, k, res, m)) || (rc = plan_launch(ctx, ws, pl, k, m, st)) ||
+        (rc = plan_finish(ctx, ws, pl, k, m, st)))
         return rc;
-    return plan_finish(ctx, ws, pl, k, m, st);
+    keep_partials(pl, m);
+    return UNG_HIP_OK;
 }
 
 int check_ready(ung_hip_ctx *ctx)
@@ -1221,7 +1336,6 @@ int cross_device(ung_hip_ctx *ctx, uint32_t G, const uint32_t *group_begin, cons
     }
     HIPCHECK(hipStreamSynchronize(ctx->ws[0].stream));
     ctx->cross.valid = true;
-    pl.part_lp = pick_lp(k, pick_lt(k), ctx->d);
     if (st)
         st->wall_ms += ms_since(t0);
     return UNG_HIP_OK;
@@ -1264,11 +1378,10 @@ int cross_intra_begin(ung_hip_ctx *ctx, uint32_t G, const uint32_t *group_begin,
     // 18.0 ms with the group select alone between the cross merge and the additional edges)
     PlanMem m0;
     if ((rc = cross_prepare_result(ctx, k)) ||
-        (rc = workspace_mem(ctx->ws[0], pl, pick_lp(k, pick_lt(k), ctx->d), ctx->cross, m0)) ||
+        (rc = workspace_mem(ctx, ctx->ws[0], pl, k, ctx->cross, m0)) ||
         (rc = plan_launch(ctx, ctx->ws[0], pl, k, m0, st)) ||
         (rc = group_prepare_result(ctx, ctx->intra_plan, list_k)) ||
-        (rc = workspace_mem(ctx->ws[1], ctx->intra_plan, pick_lp(list_k, pick_lt(list_k), ctx->d), ctx->group,
-                            ctx->intra_mem)) ||
+        (rc = workspace_mem(ctx, ctx->ws[1], ctx->intra_plan, list_k, ctx->group, ctx->intra_mem)) ||
         (rc = plan_launch(ctx, ctx->ws[1], ctx->intra_plan, list_k, ctx->intra_mem, &ctx->intra_stats,
                           ctx->ws[0].ev[1]))) {
         drain_after_failure(ctx);
@@ -1288,7 +1401,7 @@ int cross_intra_begin(ung_hip_ctx *ctx, uint32_t G, const uint32_t *group_begin,
         return rc;
     }
     ctx->cross.valid = true;
-    pl.part_lp = pick_lp(k, pick_lt(k), ctx->d);
+    keep_partials(pl, m0);
     if (st)
         st->wall_ms += ms_since(t0);
     return UNG_HIP_OK;
@@ -1446,7 +1559,6 @@ int group_device(ung_hip_ctx *ctx, uint32_t n_groups, const uint32_t *grp_begin,
         drain_after_failure(ctx);
         return rc;
     }
-    pl.part_lp = pick_lp(list_k, pick_lt(list_k), ctx->d); // partial rows kept for the diagnostics
     if (st)
         st->wall_ms += ms_since(t0);
     return UNG_HIP_OK;
@@ -1781,13 +1893,15 @@ int prepare_common(ung_hip_ctx *ctx, const float *src, bool src_device, uint64_t
     ung_hip_release_vectors(ctx);
     const auto t0 = clk::now();
     const uint32_t dp = (dim + KC - 1) / KC * KC;
+    const uint32_t hp = (dim + 2 * KC - 1) / (2 * KC) * KC; // two fp16 coordinates a word
     HIPCHECK(counted_malloc((void **)&ctx->X, N * dim * sizeof(float)));
     HIPCHECK(counted_malloc((void **)&ctx->XS, N * dp * sizeof(uint32_t)));
+    HIPCHECK(counted_malloc((void **)&ctx->XH, N * hp * sizeof(uint32_t)));
     HIPCHECK(counted_malloc((void **)&ctx->xn, N * sizeof(float)));
-    HIPCHECK(counted_malloc((void **)&ctx->maxbits, sizeof(unsigned int)));
+    HIPCHECK(counted_malloc((void **)&ctx->maxbits, 3 * sizeof(unsigned int)));
     HIPCHECK(hipMemcpyAsync(ctx->X, src, N * dim * sizeof(float),
                             src_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, ctx->stream));
-    hipLaunchKernelGGL(ung_zero_u32_kernel, dim3(1), dim3(64), 0, ctx->stream, (uint32_t *)ctx->maxbits, 1u);
+    hipLaunchKernelGGL(ung_zero_u32_kernel, dim3(1), dim3(64), 0, ctx->stream, (uint32_t *)ctx->maxbits, 3u);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(ctx->stream));
     const double h2d = ms_since(t0);
@@ -1800,12 +1914,16 @@ int prepare_common(ung_hip_ctx *ctx, const float *src, bool src_device, uint64_t
     hipLaunchKernelGGL(ung_split_kernel, dim3((unsigned)split_blocks), dim3(256), 0, ctx->stream, ctx->X, N, dim, dp,
                        ctx->XS);
     HIPCHECK(hipGetLastError());
+    hipLaunchKernelGGL(ung_half_kernel, dim3((unsigned)norm_blocks), dim3(256), 0, ctx->stream, ctx->X, N, dim, hp,
+                       ctx->XH, ctx->maxbits);
+    HIPCHECK(hipGetLastError());
     HIPCHECK(hipEventRecord(ctx->ev[5], ctx->stream));
-    unsigned int mb = 0;
-    HIPCHECK(hipMemcpyAsync(&mb, ctx->maxbits, sizeof(mb), hipMemcpyDeviceToHost, ctx->stream));
+    unsigned int mb[3] = {};
+    HIPCHECK(hipMemcpyAsync(mb, ctx->maxbits, sizeof(mb), hipMemcpyDeviceToHost, ctx->stream));
     HIPCHECK(hipStreamSynchronize(ctx->stream));
-    float mxf;
-    std::memcpy(&mxf, &mb, sizeof(mxf));
+    float mxf, res2;
+    std::memcpy(&mxf, &mb[0], sizeof(mxf));
+    std::memcpy(&res2, &mb[2], sizeof(res2));
     // the pinned staging of result downloads, once per context at set-up (not in the
     // first download's time)
     if ((rc = ctx->dl_stage.ensure(DL_PIECE * DL_SLOTS)))
@@ -1815,6 +1933,19 @@ int prepare_common(ung_hip_ctx *ctx, const float *src, bool src_device, uint64_t
     ctx->dp = dp;
     // max norm, inflated for the rounding of the norm cache
     ctx->rmax = std::sqrt((double)mxf * (1.0 + 1e-5)) * (1.0 + 1e-6);
+    // The half operands serve the pre-selection of base sets whose largest coordinate is in
+    // ung_half_kernel's range (a zero, infinite or NaN one is not) and whose rounding error
+    // is what fp16 gives (at most 2^-11 of a row's norm, below 2^-10 of the largest).
+    const uint32_t e = mb[1] >> 23;
+    ctx->hp = hp;
+    ctx->half_res = std::sqrt((double)res2) * (1.0 + 1e-6);
+    ctx->half_ok = ctx->half && e >= HALF_EMIN && e <= HALF_EMAX && ctx->half_res <= ctx->rmax * 0x1p-10;
+    if (ctx->half_ok) {
+        const uint32_t sb = half_scale_bits(e);
+        float scale;
+        std::memcpy(&scale, &sb, sizeof(scale));
+        ctx->half_s2 = scale * scale;
+    }
     ctx->cross.valid = false;
     ctx->group.valid = false;
     if (st) {
@@ -1982,8 +2113,16 @@ int cross_noalloc(ung_hip_ctx *ctx, uint32_t G, const uint32_t *group_begin, con
         st->plan_ms += ms_since(t0);
     // this device's scratch array is this call's until its last kernel has finished
     std::lock_guard<std::mutex> scratch_lock(g_scratch_call_mu[ctx->device]);
+    // the split operands' shorter partial rows serve plans too large for the half ones'
     PlanMem m;
-    if ((rc = scratch_mem(ctx, pl, pick_lp(k, pick_lt(k), ctx->d), m)))
+    pick_operands(ctx, k, false, true, m);
+    rc = scratch_mem(ctx, pl, m.lp, m);
+    if (rc && m.half) {
+        clear_error();
+        pick_operands(ctx, k, false, false, m);
+        rc = scratch_mem(ctx, pl, m.lp, m);
+    }
+    if (rc)
         return rc;
     const size_t stage_bytes = stage_layout(pl).total;
     if (ctx->noalloc_stage.size() < stage_bytes) // host memory, reused by later calls
@@ -2017,7 +2156,7 @@ int cross_noalloc(ung_hip_ctx *ctx, uint32_t G, const uint32_t *group_begin, con
 
 extern "C" {
 
-const char *ung_hip_version(void) { return "ung_hip 0.2 (gfx950, split-bf16 MFMA pre-select + exact fp32 re-rank)"; }
+const char *ung_hip_version(void) { return "ung_hip 0.3 (gfx950, certified fp16 MFMA pre-select + exact fp32 re-rank)"; }
 
 int ung_hip_create(int device, ung_hip_ctx **out)
 {
@@ -2040,6 +2179,8 @@ int ung_hip_create(int device, ung_hip_ctx **out)
         ctx->force_wide = s[0] == '1';
     if (const char *s = std::getenv("UNG_HIP_NO_QREG"))
         ctx->qreg = s[0] != '1';
+    if (const char *s = std::getenv("UNG_HIP_NO_HALF"))
+        ctx->half = s[0] != '1';
     if (const char *s = std::getenv("UNG_HIP_NO_KNN"))
         ctx->knn = s[0] != '1';
     if (const char *s = std::getenv("UNG_HIP_PRUNE_EXACT"); s && s[0] == '1')
@@ -2110,6 +2251,8 @@ int ung_hip_release_vectors(ung_hip_ctx *ctx)
         (void)hipFree(ctx->X);
     if (ctx->XS)
         (void)hipFree(ctx->XS);
+    if (ctx->XH)
+        (void)hipFree(ctx->XH);
     if (ctx->xn)
         (void)hipFree(ctx->xn);
     if (ctx->maxbits)
@@ -2117,6 +2260,9 @@ int ung_hip_release_vectors(ung_hip_ctx *ctx)
     ctx->X = nullptr;
     ctx->XS = nullptr;
     ctx->dp = 0;
+    ctx->XH = nullptr;
+    ctx->hp = 0;
+    ctx->half_ok = false;
     ctx->xn = nullptr;
     ctx->maxbits = nullptr;
     ctx->N = 0;
@@ -2660,10 +2806,12 @@ int ung_hip_debug_partial_rows(ung_hip_ctx *ctx, uint64_t capacity, uint32_t *qu
                 }
         if (pass == 0) {
             *n_entries = cnt;
+            // coef * r^2 + lin * r with r >= rmax, as one factor on r^2
+            const Operands o = operands_of(ctx, pl.part_half);
             if (eps_coef)
-                *eps_coef = eps_coef_for(ctx->d) * ctx->eps_scale;
+                *eps_coef = o.coef + (o.rmax > 0.0 ? o.lin / o.rmax : 0.0);
             if (rmax)
-                *rmax = ctx->rmax;
+                *rmax = o.rmax;
             if (cnt > capacity || (cnt > 0 && (!query || !cand || !approx))) {
                 set_error("ung_hip_debug_partial_rows: capacity %llu < %llu entries", (unsigned long long)capacity,
                           (unsigned long long)cnt);

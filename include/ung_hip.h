@@ -61,8 +61,9 @@ typedef struct ung_hip_stats {
                                 and were rescanned exactly */
     uint64_t padded_pairs;   /* pairs computed by the MFMA tiles incl. padding */
     uint64_t select_bytes;   /* operand bytes the select kernel(s) stream: per work item,
-                                its query rows and its candidate rows of the split base
-                                set (4 * dp bytes a row, dp = dim rounded up to 32) */
+                                its query rows and its candidate rows of the operand set
+                                (fp16: 2 bytes a coordinate, dim rounded up to 64; split
+                                bf16 pairs: 4 bytes, dim rounded up to 32) */
     uint64_t allocations;    /* device (hipMalloc) and pinned host (hipHostMalloc)
                                 allocations the call made (buffers grown on demand) */
 } ung_hip_stats;
@@ -270,7 +271,7 @@ int ung_hip_synchronize(ung_hip_ctx *ctx);
  * largest deviation from a host-computed product; returns 0 when it ran. */
 int ung_hip_selftest_mfma(ung_hip_ctx *ctx, double *max_abs_err);
 
-/* Diagnostic, no counterpart in the reference: the approximate (split-bf16 MFMA,
+/* Diagnostic, no counterpart in the reference: the approximate (fp16 or split-bf16 MFMA,
  * expansion-form) distances behind the context's last cross-edge call or synchronous
  * group kNN call (ung_hip_group_knn, ung_hip_group_knn_device), for checking the
  * certified error bound against exact distances.  Writes one entry per partial-row
