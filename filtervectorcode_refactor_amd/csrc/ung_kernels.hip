@@ -91,7 +91,8 @@ struct SelectParams {
     float *part_dist;
     float *part_bound;
     uint32_t n_items; // items of this launch
-    uint32_t *item_ctr; // next item to take (zeroed before the launch)
+    uint32_t *item_ctr; // next item to take: one counter, or one per XCD (zeroed before the launch)
+    uint32_t run_log2;  // log2 of the consecutive items one XCD takes (XCD_RUN_NONE: one counter)
     uint32_t lp;      // entries per partial row (approximate top-Lp)
     uint32_t x_bytes; // bytes of the split base set (buffer range of the 32-bit-offset kernels)
 };
@@ -452,6 +453,28 @@ __device__ __forceinline__ uint32_t take_item(uint32_t *ctr, uint32_t *slot)
     return *slot;
 }
 
+// The same with runs of 1 << run_log2 consecutive items per XCD (blocks b, b + 8, ... share
+// an XCD): run j of the list belongs to XCD j % 8, whose blocks take its items through their
+// own counter; where an XCD has no item left its blocks take the other XCDs'.  A counter
+// hands out ascending positions, so one position past the list ends it, and n_items blocks
+// meet n_items positions (n_items <= 2^28: positions stay below 2^32).  Which XCD a block really runs on changes the speed alone.
+constexpr uint32_t N_XCD = 8;
+constexpr uint32_t XCD_RUN_NONE = 32;
+__device__ __forceinline__ uint32_t take_item_run(uint32_t *ctr, uint32_t run_log2, uint32_t n_items, uint32_t *slot)
+{
+    if (threadIdx.x == 0) {
+        uint32_t pos = n_items;
+        for (uint32_t t = 0; t < N_XCD && pos >= n_items; ++t) {
+            const uint32_t x = (blockIdx.x + t) % N_XCD;
+            const uint32_t c = atomicAdd(ctr + x, 1u);
+            pos = (((c >> run_log2) * N_XCD + x) << run_log2) + (c & ((1u << run_log2) - 1u));
+        }
+        *slot = pos;
+    }
+    __syncthreads();
+    return *slot;
+}
+
 // Pre-filter bound in s-space: s = |x|^2/2 - <x,q> and a = fl(2s + |q|^2).  Returns c
 // with  s >= c  =>  a >= thr  (the margin covers the rounding of 2s + |q|^2), so a
 // candidate failing s < c can never pass the exact test a < thr.
@@ -728,7 +751,9 @@ __global__ __launch_bounds__(select_threads<NB>(), (LT <= 8 ? 2 : 1)) void ung_s
     };
     __shared__ typename std::conditional<(LT >= 16), Tau4, NoStage>::type tau4;
     __shared__ uint32_t item_slot;
-    const uint32_t logical = take_item(P.item_ctr, &item_slot);
+    const uint32_t logical = !QR && P.run_log2 != XCD_RUN_NONE
+                                 ? take_item_run(P.item_ctr, P.run_log2, P.n_items, &item_slot)
+                                 : take_item(P.item_ctr, &item_slot);
     if (logical >= P.n_items)
         return;
     const Item it = P.items[logical];

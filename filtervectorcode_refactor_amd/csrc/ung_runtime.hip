@@ -209,7 +209,7 @@ struct PlanMem {
     uint32_t *seg_start = nullptr, *seg_vend = nullptr;
     uint32_t *part_ids = nullptr;
     float *part_dist = nullptr, *part_bound = nullptr;
-    uint32_t *flag_count = nullptr; // [0]: rows flagged for the rescan, [1]: select item counter
+    uint32_t *flag_count = nullptr; // [0]: rows flagged for the rescan, then the select's item counters
     uint2 *flagged = nullptr;
     uint2 *tiny = nullptr;          // Plan::tiny
     uint32_t *out_ids = nullptr;    // result rows
@@ -243,7 +243,7 @@ struct Workspace {
     DevBuf<uint32_t> part_ids;
     DevBuf<float> part_dist;
     DevBuf<float> part_bound;
-    DevBuf<uint32_t> flag_count; // [0]: rows flagged for the rescan, [1]: select item counter
+    DevBuf<uint32_t> flag_count; // [0]: rows flagged for the rescan, then the select's item counters
     DevBuf<uint2> flagged;
     DevBuf<uint2> tiny;
     DevBuf<uint32_t> fb_ids; // rescan range results
@@ -372,6 +372,36 @@ uint32_t split_size(uint64_t u)
     return (uint32_t)std::max<uint64_t>(SPLIT_V, s);
 }
 
+// Half operand rows (hp words) so long that the query panels of an XCD's 64 resident blocks,
+// re-read for every candidate tile, take several times its 4 MB L2 (16 KB panels at d = 64;
+// from d = 449 on, 8 MB and more).  Such a select is bound by what it fetches past the L2
+// (2M x 768: 7.4 TB/s), so the blocks of one XCD take runs of 64 consecutive items
+// (take_item_run) and the cross plan's runs are all splits of a few query blocks.
+// Measured at both sides: 2M x 768 select 76.6 -> 71.2 ms (runs alone 75.0), lists of 10
+// groups at 400k x 768 4.73 -> 4.37 ms (runs of 32: 4.74); 1M x 384 8.05 -> 8.60 ms, whose
+// operands mostly hit the L2 (20 GB fetched) and whose few long items a run puts on one XCD.
+bool long_rows(uint32_t hp) { return (uint64_t)hp * sizeof(uint32_t) * BQ * 64u >= (8ull << 20); }
+constexpr uint32_t LONG_RUN_LOG2 = 6;
+
+// Candidates per split of a cross job of u candidates with long rows: up to 4 splits of at
+// least 2048 candidates (16 tiles).  8 splits: select 69.7 ms, but merge 5.1 -> 6.9 ms.
+constexpr uint64_t FINE_SPLITS = 4, FINE_SPLIT_MIN = 2048;
+uint32_t split_size_cross(uint64_t u, bool fine)
+{
+    const uint32_t coarse = split_size(u);
+    if (!fine)
+        return coarse;
+    const uint64_t ns = std::min<uint64_t>(FINE_SPLITS, std::max<uint64_t>(1, u / FINE_SPLIT_MIN));
+    return (uint32_t)std::min<uint64_t>(coarse, ((u + ns - 1) / ns + BC - 1) / BC * BC);
+}
+
+// Fine splits only up to 8M rows: at most 4 splits x 80 entries x 8 bytes a row of partial
+// rows (16 entries at k = 6), which larger base sets may not have to spare.
+bool fine_splits(const ung_hip_ctx *ctx)
+{
+    return ctx->half_ok && long_rows(ctx->hp) && ctx->N <= (1ull << 23);
+}
+
 // Empties a plan, keeping the capacity of its lists.
 void plan_reset(Plan &pl)
 {
@@ -491,7 +521,7 @@ int launch_items(ung_hip_ctx *ctx, hipStream_t stream, const SelectParams &P, ui
         Q.x_bytes = mode == LOAD_BUF32 ? (uint32_t)(ctx->N * P.dp * sizeof(uint32_t)) : 0u;
         Q.n_items = std::min(max_grid, n_items - off);
         if (off > 0) { // the counter was zeroed for the first chunk by the caller
-            hipLaunchKernelGGL(ung_zero_u32_kernel, dim3(1), dim3(64), 0, stream, P.item_ctr, 1u);
+            hipLaunchKernelGGL(ung_zero_u32_kernel, dim3(1), dim3(64), 0, stream, P.item_ctr, N_XCD);
             HIPCHECK(hipGetLastError());
         }
         hipLaunchKernelGGL(kernel, dim3(Q.n_items), dim3(threads), 0, stream, Q);
@@ -507,6 +537,8 @@ int launch_select_t(ung_hip_ctx *ctx, hipStream_t stream, const SelectParams &P,
     // queues longer than 8 take the one-column-per-lane layout (two waves per SIMD)
     constexpr int NB = LT <= 8 ? 2 : 1;
     const int th = select_threads<NB>();
+    SelectParams R = P;
+    R.run_log2 = HALF && long_rows(P.dp) && n_items <= (1u << 28) ? LONG_RUN_LOG2 : XCD_RUN_NONE;
     if constexpr (NB == 2 && HALF) {
         // two columns per lane and half operands of 128 dimensions: the register-query layout
         if (P.dp == (uint32_t)(QR_NK * KC) && ctx->qreg) {
@@ -518,10 +550,10 @@ int launch_select_t(ung_hip_ctx *ctx, hipStream_t stream, const SelectParams &P,
         }
     }
     if (mode == LOAD_BUF32)
-        return excl ? launch_items(ctx, stream, P, n_items, mode, th, ung_select_kernel<LT, LOAD_BUF32, true, NB, false, HALF>)
-                    : launch_items(ctx, stream, P, n_items, mode, th, ung_select_kernel<LT, LOAD_BUF32, false, NB, false, HALF>);
-    return excl ? launch_items(ctx, stream, P, n_items, mode, th, ung_select_kernel<LT, LOAD_WIDE, true, NB, false, HALF>)
-                : launch_items(ctx, stream, P, n_items, mode, th, ung_select_kernel<LT, LOAD_WIDE, false, NB, false, HALF>);
+        return excl ? launch_items(ctx, stream, R, n_items, mode, th, ung_select_kernel<LT, LOAD_BUF32, true, NB, false, HALF>)
+                    : launch_items(ctx, stream, R, n_items, mode, th, ung_select_kernel<LT, LOAD_BUF32, false, NB, false, HALF>);
+    return excl ? launch_items(ctx, stream, R, n_items, mode, th, ung_select_kernel<LT, LOAD_WIDE, true, NB, false, HALF>)
+                : launch_items(ctx, stream, R, n_items, mode, th, ung_select_kernel<LT, LOAD_WIDE, false, NB, false, HALF>);
 }
 
 template <bool HALF>
@@ -644,7 +676,7 @@ int workspace_mem(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, R
         (rc = ws.mitems.ensure(pl.n_mitems)) || (rc = ws.seg_start.ensure(pl.seg_start.size())) ||
         (rc = ws.seg_vend.ensure(pl.seg_vend.size())) ||
         (rc = ws.part_ids.ensure(pl.part_rows * lp)) || (rc = ws.part_dist.ensure(pl.part_rows * lp)) ||
-        (rc = ws.part_bound.ensure(pl.part_rows)) || (rc = ws.flag_count.ensure(2)) ||
+        (rc = ws.part_bound.ensure(pl.part_rows)) || (rc = ws.flag_count.ensure(1 + N_XCD)) ||
         (rc = ws.flagged.ensure(std::max<uint64_t>(pl.rows, 1))) || (rc = ws.tiny.ensure(pl.n_tiny + 1)))
         return rc;
     if (!pl.jobs.empty()) {
@@ -818,7 +850,7 @@ int plan_launch(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, Pla
 int plan_launch_select(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, PlanMem &m)
 {
     int rc;
-    hipLaunchKernelGGL(ung_zero_u32_kernel, dim3(1), dim3(64), 0, ws.stream, m.flag_count, 2u);
+    hipLaunchKernelGGL(ung_zero_u32_kernel, dim3(1), dim3(64), 0, ws.stream, m.flag_count, 1u + N_XCD);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipEventRecord(ws.ev[0], ws.stream));
 
@@ -839,6 +871,7 @@ int plan_launch_select(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t
     P.part_dist = m.part_dist;
     P.part_bound = m.part_bound;
     P.item_ctr = m.flag_count + 1;
+    P.run_log2 = XCD_RUN_NONE;
     P.lp = lp;
     const uint32_t n_items = (uint32_t)pl.items.size();
     const bool excl = (pl.jobs[0].flags & 1u) != 0; // one kind of job per plan
@@ -1085,7 +1118,7 @@ struct PlanChunk {
 // (the out-groups' ranges in LNG row order), and its items (query blocks x splits,
 // split-major).  Two passes over chunks of groups on the context's worker pool.
 int build_cross_plan(ung_hip_ctx *ctx, uint32_t G, const uint32_t *group_begin, const uint32_t *out_ptr,
-                     const uint32_t *out_idx, Plan &pl)
+                     const uint32_t *out_idx, Plan &pl, bool fine)
 {
     if (!group_begin || !out_ptr || (out_ptr[G + 1] > 0 && !out_idx)) {
         set_error("ung_hip_cross_topk: null group_begin/out_ptr/out_idx");
@@ -1162,7 +1195,7 @@ int build_cross_plan(ung_hip_ctx *ctx, uint32_t G, const uint32_t *group_begin, 
                 c.tiny += 1;
                 continue;
             }
-            const uint64_t sv = split_size(u), ns = (u + sv - 1) / sv, qb = (qn + BQ - 1) / BQ;
+            const uint64_t sv = split_size_cross(u, fine), ns = (u + sv - 1) / sv, qb = (qn + BQ - 1) / BQ;
             c.items += ns * qb;
             c.mitems += (qn + MERGE_ROWS - 1) / MERGE_ROWS;
             c.part_rows += (uint64_t)qn * ns;
@@ -1244,23 +1277,26 @@ int build_cross_plan(ung_hip_ctx *ctx, uint32_t G, const uint32_t *group_begin, 
                 ++j;
                 continue;
             }
-            jb.split_v = split_size(u);
+            jb.split_v = split_size_cross(u, fine);
             jb.n_split = (uint32_t)((u + jb.split_v - 1) / jb.split_v);
             jb.part_base = (uint32_t)part;
             part += (uint64_t)qn * jb.n_split;
             pl.jobs[j] = jb;
-            // split-major: consecutive items are query blocks streaming the same candidates
-            for (uint32_t s = 0; s < jb.n_split; ++s)
-                for (uint32_t qo = 0; qo < qn; qo += BQ) {
-                    Item it{};
-                    it.job = (uint32_t)j;
-                    it.q_off = qo;
-                    it.q_cnt = std::min<uint32_t>(BQ, qn - qo);
-                    it.v_begin = s * jb.split_v;
-                    it.v_end = (uint32_t)std::min<uint64_t>(u, (uint64_t)(s + 1) * jb.split_v);
-                    it.split = s;
-                    pl.items[itn++] = it;
-                }
+            // split-major: consecutive items are query blocks streaming the same candidates;
+            // fine: query-major, all splits of a query block
+            const uint32_t qb = (qn + BQ - 1) / BQ;
+            for (uint32_t i = 0; i < jb.n_split * qb; ++i) {
+                const uint32_t s = fine ? i % jb.n_split : i / qb;
+                const uint32_t qo = (fine ? i / jb.n_split : i % qb) * BQ;
+                Item it{};
+                it.job = (uint32_t)j;
+                it.q_off = qo;
+                it.q_cnt = std::min<uint32_t>(BQ, qn - qo);
+                it.v_begin = s * jb.split_v;
+                it.v_end = (uint32_t)std::min<uint64_t>(u, (uint64_t)(s + 1) * jb.split_v);
+                it.split = s;
+                pl.items[itn++] = it;
+            }
             ++j;
         }
     };
@@ -1326,7 +1362,7 @@ int cross_device(ung_hip_ctx *ctx, uint32_t G, const uint32_t *group_begin, cons
     const auto t0 = clk::now();
     Plan &pl = ctx->plan0;
     plan_reset(pl);
-    if ((rc = build_cross_plan(ctx, G, group_begin, out_ptr, out_idx, pl)))
+    if ((rc = build_cross_plan(ctx, G, group_begin, out_ptr, out_idx, pl, fine_splits(ctx))))
         return rc;
     if (st)
         st->plan_ms += ms_since(t0);
@@ -1360,7 +1396,7 @@ int cross_intra_begin(ung_hip_ctx *ctx, uint32_t G, const uint32_t *group_begin,
     const auto t0 = clk::now();
     Plan &pl = ctx->plan0;
     plan_reset(pl);
-    if ((rc = build_cross_plan(ctx, G, group_begin, out_ptr, out_idx, pl)))
+    if ((rc = build_cross_plan(ctx, G, group_begin, out_ptr, out_idx, pl, fine_splits(ctx))))
         return rc;
     if (st)
         st->plan_ms += ms_since(t0);
@@ -2020,7 +2056,7 @@ int scratch_mem(ung_hip_ctx *ctx, const Plan &pl, uint32_t lp, PlanMem &m)
     const uint64_t o_pid = take(pl.part_rows * lp * sizeof(uint32_t));
     const uint64_t o_pd = take(pl.part_rows * lp * sizeof(float));
     const uint64_t o_pb = take(pl.part_rows * sizeof(float));
-    const uint64_t o_fc = take(2 * sizeof(uint32_t));
+    const uint64_t o_fc = take((1 + N_XCD) * sizeof(uint32_t));
     const uint64_t o_fl = take(std::max<uint64_t>(pl.rows, 1) * sizeof(uint2));
     const uint64_t o_tiny = take((pl.n_tiny + 1) * sizeof(uint2));
     if (off > UNG_HIP_NOALLOC_SCRATCH_BYTES) {
@@ -2107,7 +2143,7 @@ int cross_noalloc(ung_hip_ctx *ctx, uint32_t G, const uint32_t *group_begin, con
     ctx->cross.rescanned.clear();
     Plan &pl = ctx->plan0;
     plan_reset(pl);
-    if ((rc = build_cross_plan(ctx, G, group_begin, out_ptr, out_idx, pl)))
+    if ((rc = build_cross_plan(ctx, G, group_begin, out_ptr, out_idx, pl, false))) // (no more scratch than it has to)
         return rc;
     if (st)
         st->plan_ms += ms_since(t0);
