@@ -279,7 +279,7 @@ struct ung_hip_ctx {
     uint32_t dp = 0;        // its row pitch in words
     uint32_t *XH = nullptr; // half base set (scaled fp16) for the MFMA pre-selection
     uint32_t hp = 0;        // its row pitch in words
-    bool half_ok = false;   // XH is usable (half_rule)
+    bool half_ok = false;   // XH is usable (prepare_common)
     float half_s2 = 1.0f;   // its squared scale
     double half_res = 0.0;  // largest norm of what the fp16 rounding left out of a row (rounded up)
     float *xn = nullptr;
@@ -1932,9 +1932,17 @@ int prepare_common(ung_hip_ctx *ctx, const float *src, bool src_device, uint64_t
     const uint32_t hp = (dim + 2 * KC - 1) / (2 * KC) * KC; // two fp16 coordinates a word
     HIPCHECK(counted_malloc((void **)&ctx->X, N * dim * sizeof(float)));
     HIPCHECK(counted_malloc((void **)&ctx->XS, N * dp * sizeof(uint32_t)));
-    HIPCHECK(counted_malloc((void **)&ctx->XH, N * hp * sizeof(uint32_t)));
     HIPCHECK(counted_malloc((void **)&ctx->xn, N * sizeof(float)));
     HIPCHECK(counted_malloc((void **)&ctx->maxbits, 3 * sizeof(unsigned int)));
+    // The half set only where it leaves an eighth of the device memory for results and
+    // workspaces: a base set that fits without it is served by the split operands.
+    size_t mem_free = 0, mem_total = 0;
+    HIPCHECK(hipMemGetInfo(&mem_free, &mem_total));
+    if (N * hp * sizeof(uint32_t) + mem_total / 8 <= mem_free &&
+        counted_malloc((void **)&ctx->XH, N * hp * sizeof(uint32_t)) != hipSuccess) {
+        (void)hipGetLastError();
+        ctx->XH = nullptr;
+    }
     HIPCHECK(hipMemcpyAsync(ctx->X, src, N * dim * sizeof(float),
                             src_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, ctx->stream));
     hipLaunchKernelGGL(ung_zero_u32_kernel, dim3(1), dim3(64), 0, ctx->stream, (uint32_t *)ctx->maxbits, 3u);
@@ -1950,9 +1958,11 @@ int prepare_common(ung_hip_ctx *ctx, const float *src, bool src_device, uint64_t
     hipLaunchKernelGGL(ung_split_kernel, dim3((unsigned)split_blocks), dim3(256), 0, ctx->stream, ctx->X, N, dim, dp,
                        ctx->XS);
     HIPCHECK(hipGetLastError());
-    hipLaunchKernelGGL(ung_half_kernel, dim3((unsigned)norm_blocks), dim3(256), 0, ctx->stream, ctx->X, N, dim, hp,
-                       ctx->XH, ctx->maxbits);
-    HIPCHECK(hipGetLastError());
+    if (ctx->XH) {
+        hipLaunchKernelGGL(ung_half_kernel, dim3((unsigned)norm_blocks), dim3(256), 0, ctx->stream, ctx->X, N, dim, hp,
+                           ctx->XH, ctx->maxbits);
+        HIPCHECK(hipGetLastError());
+    }
     HIPCHECK(hipEventRecord(ctx->ev[5], ctx->stream));
     unsigned int mb[3] = {};
     HIPCHECK(hipMemcpyAsync(mb, ctx->maxbits, sizeof(mb), hipMemcpyDeviceToHost, ctx->stream));
@@ -1975,7 +1985,7 @@ int prepare_common(ung_hip_ctx *ctx, const float *src, bool src_device, uint64_t
     const uint32_t e = mb[1] >> 23;
     ctx->hp = hp;
     ctx->half_res = std::sqrt((double)res2) * (1.0 + 1e-6);
-    ctx->half_ok = ctx->half && e >= HALF_EMIN && e <= HALF_EMAX && ctx->half_res <= ctx->rmax * 0x1p-10;
+    ctx->half_ok = ctx->half && ctx->XH && e >= HALF_EMIN && e <= HALF_EMAX && ctx->half_res <= ctx->rmax * 0x1p-10;
     if (ctx->half_ok) {
         const uint32_t sb = half_scale_bits(e);
         float scale;
