@@ -41,7 +41,7 @@ import numpy as np
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
-MFMA_BF16_PEAK_TFLOPS = 2500.0  # dense
+MFMA_16BIT_PEAK_TFLOPS = 2500.0  # dense
 MFMA_FP32_PEAK_TFLOPS = 157.3
 HBM_PEAK_GBS = 8000.0
 METRIC = "cross-edge build wall time + distance evals/s (MFMA util %), 1M×128 fp32, 1 GPU"
@@ -181,7 +181,7 @@ def cpu_leg_and_parity(st, cfg, gpu_cross, gpu_intra, p_cross, p_intra, seconds,
     # keeps k+1 entries so the k-th / (k+1)-th boundary can be checked for the tie band
     def cross_run(q):
         t0 = time.perf_counter()
-        ri, rd = ref.cross_exact_points(st.base, st.group_begin, pg, st.out_ptr, st.out_idx, q, k + 1, threads)
+        ri, rd = ref.cross_exact_points(st.base, st.group_begin, pg, st.out_ptr, st.out_idx, q, k + 1, threads)[:2]
         return ri, rd, time.perf_counter() - t0
 
     budget_x = seconds * 2 / 3 if timed else 0.0
@@ -237,7 +237,8 @@ def cpu_leg_and_parity(st, cfg, gpu_cross, gpu_intra, p_cross, p_intra, seconds,
         "tie_band_kth_boundary_rows": boundary_x,
         "tie_band": f"adjacent entries of the reference's sorted rows (cross: top-{k + 1}, intra: top-{K}) within "
                     f"{TIE_BAND:g} relative; kth_boundary = cross rows whose {k}-th and {k + 1}-th differ by at most that",
-        "checker": f"oracle/_ref ({kind}: the reference's compiled distance.cpp + search_queue.cpp scan)",
+        "checker": ("oracle/_ref (the reference's compiled distance.cpp + search_queue.cpp scan)" if kind == "reference"
+                    else "the plain-C oracle's exact scan"),
     }
     if not timed:
         return None, parity
@@ -373,17 +374,17 @@ def main():
     sel_cross_ms = avg(cross_stats, "select_ms")
     sel_intra_ms = avg(intra_stats, "select_ms")
     d = cfg.dim
-    dp = (d + 31) // 32 * 32
-    # The cross select kernel's two floors: its MFMA work (three bf16 products per fp32
-    # product: 3 * 2 * dp flops per algorithmic pair, against the dense bf16 peak) and its
+    dp = (d + 63) // 64 * 64  # dimensions of an operand row
+    # The cross select kernel's two floors: its MFMA work (one fp16 product per
+    # coordinate pair: 2 * dp flops per algorithmic pair, against the dense 16-bit peak) and its
     # HBM traffic (measured with rocprofv3 on this kernel source, against 8 TB/s).  The
     # larger floor bounds it; without a valid traffic measurement the MFMA floor is used.
     sel_s = sel_cross_ms * 1e-3
     flops_cross = 2.0 * d * p_cross
-    mfma_flops = 3.0 * 2.0 * dp * p_cross
+    mfma_flops = 2.0 * dp * p_cross
     alg_bytes = float(cross_stats[-1]["select_bytes"])
     traffic, traffic_status = read_traffic(cfg.name) if not args.n else (None, "not measured (scaled run)")
-    mfma_floor_ms = mfma_flops / (MFMA_BF16_PEAK_TFLOPS * 1e12) * 1e3
+    mfma_floor_ms = mfma_flops / (MFMA_16BIT_PEAK_TFLOPS * 1e12) * 1e3
     hbm_floor_ms = traffic / (HBM_PEAK_GBS * 1e9) * 1e3 if traffic else None
     mfma_tflops = mfma_flops / sel_s / 1e12
     if hbm_floor_ms is not None and hbm_floor_ms >= mfma_floor_ms:
@@ -391,17 +392,17 @@ def main():
         roofline = {"bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                     "frac": round(ach / HBM_PEAK_GBS, 4), "traffic": traffic}
     else:
-        roofline = {"bound": "mfma", "achieved": round(mfma_tflops, 3), "peak": MFMA_BF16_PEAK_TFLOPS,
-                    "unit": "TFLOP/s", "frac": round(mfma_tflops / MFMA_BF16_PEAK_TFLOPS, 4), "traffic": traffic}
+        roofline = {"bound": "mfma", "achieved": round(mfma_tflops, 3), "peak": MFMA_16BIT_PEAK_TFLOPS,
+                    "unit": "TFLOP/s", "frac": round(mfma_tflops / MFMA_16BIT_PEAK_TFLOPS, 4), "traffic": traffic}
     roofline.update({
-        "kernel": ("ung_select_kernel<8,*,false,2,true> (cross edges, register-query layout, one launch per step)"
-                   if dp == 128 else "ung_select_kernel<8,*,false,2,false> (cross edges, one launch per step)"),
+        "kernel": ("ung_select_kernel<8,*,false,2,true,true> (cross edges, register-query layout, one launch per step)"
+                   if dp == 128 else "ung_select_kernel<8,*,false,2,false,true> (cross edges, one launch per step)"),
         "avg_launch_ms": round(sel_cross_ms, 4),
         "traffic_status": traffic_status,
         "streamed_operand_bytes_per_launch": alg_bytes,
         "hbm_floor_ms": round(hbm_floor_ms, 3) if hbm_floor_ms is not None else None,
-        "mfma_bf16_flops_per_launch": mfma_flops, "mfma_floor_ms": round(mfma_floor_ms, 3),
-        "mfma_bf16_tflops": round(mfma_tflops, 2), "mfma_bf16_frac": round(mfma_tflops / MFMA_BF16_PEAK_TFLOPS, 4),
+        "mfma_flops_per_launch": mfma_flops, "mfma_floor_ms": round(mfma_floor_ms, 3),
+        "mfma_tflops": round(mfma_tflops, 2), "mfma_frac": round(mfma_tflops / MFMA_16BIT_PEAK_TFLOPS, 4),
         "measured_hbm_gbs": round(traffic / sel_s / 1e9, 1) if traffic else None,
         "fp32_equiv_tflops": round(flops_cross / sel_s / 1e12, 2),
     })
@@ -410,7 +411,7 @@ def main():
         "metric": METRIC, "value": value, "unit": "distance evals/s", "n_gpus": 1,
         "steps": steps, "warmup": warmup, "ms_per_step": round(ms_per_step, 3),
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-        "dtype": "f32 (3xbf16 MFMA pre-select, exact f32 re-score)",
+        "dtype": "f32 (certified fp16 MFMA pre-select, exact f32 re-score)",
         "data": "synthetic",
         "config": {"workload": f"{cfg.name}: {cfg.n}x{cfg.dim} fp32 Gaussian mixture "
                                f"({cfg.n_centroids} centroids, sigma {cfg.sigma}), vocab {cfg.vocab}, "

@@ -37,7 +37,7 @@ PASSES = {
 }
 N_XCD = 8            # GRBM_GUI_ACTIVE adds the busy cycles of the eight XCDs
 N_SIMD = 256 * 4     # SIMDs of the MI355X
-BF16_PEAK = 2.5e15
+MFMA_PEAK = 2.5e15
 
 
 def _short(name: str) -> str:
@@ -68,7 +68,7 @@ def trace(cfg: str, d: str):
     timed = sel[warm: warm + steps]
     dur = [(int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e6 for r in timed]
     tavg = sum(dur) / len(dur)
-    f = rl["mfma_bf16_flops_per_launch"]
+    f = rl["mfma_flops_per_launch"]
     out = [f"# Kernel trace — {cfg} ({C.n:,} x {C.dim} fp32, cross k={C.k_cross} + intra K={C.k_intra}), MI355X", "",
            "Command (from the repository root on the MI355X box):", "",
            f"    rocprofv3 --kernel-trace --stats --output-format csv -d gpurun_out/meas/{cfg}/trace -o t -- \\",
@@ -85,8 +85,8 @@ def trace(cfg: str, d: str):
             f"{tavg:.3f} ms on average (min {min(dur):.3f}, max {max(dur):.3f}); the bench's HIP-event average of the "
             f"same launches (`roofline.avg_launch_ms`) is {rl['avg_launch_ms']:.3f} ms "
             f"({abs(tavg - rl['avg_launch_ms']) / rl['avg_launch_ms'] * 100:.1f} % apart).",
-            f"Per launch: 3 bf16 MFMA passes, 2 * 3 * dp * P_cross = {f:.4g} FLOP: {f / tavg / 1e9:.0f} TFLOP/s from the "
-            f"trace = {f / tavg / 1e9 / (BF16_PEAK / 1e12) * 100:.1f} % of the 2.5 PFLOP/s dense bf16 peak; the line's "
+            f"Per launch: one fp16 MFMA pass, 2 * dp * P_cross = {f:.4g} FLOP: {f / tavg / 1e9:.0f} TFLOP/s from the "
+            f"trace = {f / tavg / 1e9 / (MFMA_PEAK / 1e12) * 100:.1f} % of the 2.5 PFLOP/s dense 16-bit peak; the line's "
             f"`roofline` ({rl['bound']}) frac is {rl['frac']}."]
     out += ["", f"Bench line of this run: ms_per_step {B['ms_per_step']}, value {B['value']:.4g} {B['unit']}; "
             f"cross select {bd['cross_select_ms']} ms, merge {bd['cross_merge_ms']} ms, additional edges "
