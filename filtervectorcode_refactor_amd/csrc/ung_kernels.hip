@@ -419,17 +419,33 @@ struct alignas(16) SelectSmem {
 };
 static_assert(BQ == BC, "the epilogue staging addresses assume square panels");
 
-// Register-query layout (half operand rows of 128 dimensions, two query columns per lane): a
+// Register-query layout (operand rows of 128 dimensions, two query columns per lane): a
 // lane keeps its query columns' operands of all 8 k-blocks in registers for the whole item;
-// per step only the candidate chunk is loaded and staged.  Select 1M x 128: 8.5 ms, bound by
-// the epilogue's VALU work (51 % of the SIMD cycles, MFMA 30 %).  One query column a lane
-// (8 waves a block, four a SIMD) takes 9.0 ms.
-constexpr int QR_NK = 2; // chunks of 64 dimensions
+// per step only the candidate chunk is loaded and staged.  Of the split operands it keeps the
+// high words; the low words of the item's queries stay in LDS.
+//   half:  select 1M x 128 8.5 ms, bound by the epilogue's VALU work (51 % of the SIMD cycles,
+//          MFMA 30 %); one query column a lane (8 waves a block, four a SIMD) takes 9.0 ms;
+//   split: 13.9 ms, with both panels restaged every step 18.1 ms (LDS traffic per step and
+//          wave 16 KB against 24 KB).
+template <bool HALF>
+constexpr int qr_chunks() // chunks of 64 (half) or 32 (split) dimensions
+{
+    return HALF ? 2 : 4;
+}
+constexpr int QLO_W = qr_chunks<false>() * 16 + 4; // words per resident low-word query row (padded)
+template <bool HALF>
+struct SelectPanelsQ {
+    float4 xs[2][BC][LDSW / 4];
+};
+template <>
+struct SelectPanelsQ<false> {
+    float4 xs[2][BC][LDSW / 4];
+    float4 qlo[BQ][QLO_W / 4];
+};
+template <bool HALF>
 struct alignas(16) SelectSmemQ {
     union {
-        struct {
-            float4 xs[2][BC][LDSW / 4];
-        } p;
+        SelectPanelsQ<HALF> p;
         SelectRed r;
     } u;
     uint32_t rowid[3][BC];
@@ -738,13 +754,15 @@ template <int LT, int MODE, bool EXCL, int NB, bool QR, bool HALF>
 __global__ __launch_bounds__(select_threads<NB>(), (LT <= 8 ? 2 : 1)) void ung_select_kernel(SelectParams P)
 {
     static_assert(NB == 1 || NB == 2, "one or two query columns per lane");
-    static_assert(!QR || (NB == 2 && LT == 8 && HALF), "register-query layout: NB = 2, LT = 8, half operands");
+    static_assert(!QR || (NB == 2 && LT == 8), "register-query layout: NB = 2, LT = 8");
+    constexpr int QR_NK = qr_chunks<HALF>();
+    constexpr int NKB = HALF ? 4 : 2; // k-blocks of 16 dimensions per chunk
     constexpr int NTH = select_threads<NB>();
     constexpr int WN = 4 / NB;         // query waves
     constexpr int QW = 32 * NB;        // query columns per wave
     constexpr int RSTEP = NTH / 8;     // loader row step
     constexpr int LM = BQ / RSTEP;     // rows per thread and panel
-    __shared__ typename std::conditional<QR, SelectSmemQ, SelectSmem>::type sm;
+    __shared__ typename std::conditional<QR, SelectSmemQ<HALF>, SelectSmem>::type sm;
     __shared__ typename std::conditional<NB == 1, SelectStage, NoStage>::type stage;
     // long queues: [tile parity][candidate wave][query] the larger m4-th entry of a wave's
     // two queues of the query
@@ -820,17 +838,29 @@ __global__ __launch_bounds__(select_threads<NB>(), (LT <= 8 ? 2 : 1)) void ung_s
     const uint32_t qoff = ((uint32_t)lr0 * dp + (uint32_t)c4) * 4u;
 
     // register-query layout: this lane's query columns, one float4 per k-block of 16
-    // dimensions (k-block kb: words 8 kb + 4 h .. +3 of the row)
-    [[maybe_unused]] halfx8 bhr[4 * QR_NK][NB];
+    // dimensions.  half: k-block kb in words 8 kb + 4 h .. +3 of the row; split: its high words
+    // in float4 column 2*(kb%2) + h of chunk kb/2, the low words of all the item's queries
+    // (float4 column 4*chunk + c of row q) in LDS
+    [[maybe_unused]] u32x4 bhr[NKB * QR_NK][NB];
     if constexpr (QR) {
         // rows of the item's queries (row 0 of qres is query q0; zeros past its qcnt rows)
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
             const uint32_t row = (uint32_t)(wn * QW + 32 * nb + r);
 #pragma unroll
-            for (int kb = 0; kb < 4 * QR_NK; ++kb)
-                bhr[kb][nb] = __builtin_bit_cast(
-                    halfx8, __builtin_amdgcn_raw_buffer_load_b128(qres, (row * dp + (uint32_t)(8 * kb + 4 * h)) * 4u, 0, 0));
+            for (int kb = 0; kb < NKB * QR_NK; ++kb) {
+                const int w = HALF ? 8 * kb + 4 * h : (kb >> 1) * KC + (2 * (kb & 1) + h) * 4;
+                bhr[kb][nb] = __builtin_amdgcn_raw_buffer_load_b128(qres, (row * dp + (uint32_t)w) * 4u, 0, 0);
+            }
+        }
+        if constexpr (!HALF) {
+#pragma unroll
+            for (int i = 0; i < BQ * QR_NK * 4 / NTH; ++i) {
+                const int idx = tid + NTH * i;
+                const int q = idx >> 4, f = idx & 15; // f = 4*chunk + float4 column of the low words
+                const uint32_t off = ((uint32_t)q * dp + (uint32_t)((f >> 2) * KC + 16 + (f & 3) * 4)) * 4u;
+                sm.u.p.qlo[q][f] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(qres, off, 0, 0));
+            }
         }
     }
 
@@ -928,72 +958,73 @@ __global__ __launch_bounds__(select_threads<NB>(), (LT <= 8 ? 2 : 1)) void ung_s
         auto mfma_chunk = [&](auto first_chunk) {
             constexpr bool FIRST = decltype(first_chunk)::value;
             const floatx16 zero = {};
-            if constexpr (HALF) {
+            // float4 column ch of this wave's query rows of the chunk (QR: their registers)
+            auto query = [&](int nb, int kb, int ch) __attribute__((always_inline)) {
+                if constexpr (QR)
+                    return bhr[NKB * decltype(kcv)::value + kb][nb];
+                else
+                    return __builtin_bit_cast(u32x4, sm.u.p.qs[buf][wn * QW + 32 * nb + r][ch]);
+            };
 #pragma unroll
-                for (int kb = 0; kb < 4; ++kb) {
-                    const int ch = 2 * kb + h;
+            for (int kb = 0; kb < NKB; ++kb) {
+                const int ch = 2 * kb + h; // float4 column (split: of the high parts; +4: low parts)
+                const bool z = FIRST && kb == 0;
+                if constexpr (HALF) {
                     halfx8 a[2], b[NB];
 #pragma unroll
                     for (int mb = 0; mb < 2; ++mb)
                         a[mb] = __builtin_bit_cast(halfx8, sm.u.p.xs[buf][wm * 64 + 32 * mb + r][ch]);
 #pragma unroll
+                    for (int nb = 0; nb < NB; ++nb)
+                        b[nb] = __builtin_bit_cast(halfx8, query(nb, kb, ch));
+#pragma unroll
+                    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+                        for (int nb = 0; nb < NB; ++nb)
+                            acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[mb], b[nb], z ? zero : acc[mb][nb], 0, 0, 0);
+                } else {
+                    bf16x8 ah[2], al[2], bh[NB], bl[NB];
+#pragma unroll
+                    for (int mb = 0; mb < 2; ++mb) {
+                        ah[mb] = __builtin_bit_cast(bf16x8, sm.u.p.xs[buf][wm * 64 + 32 * mb + r][ch]);
+                        al[mb] = __builtin_bit_cast(bf16x8, sm.u.p.xs[buf][wm * 64 + 32 * mb + r][ch + 4]);
+                    }
+#pragma unroll
                     for (int nb = 0; nb < NB; ++nb) {
+                        bh[nb] = __builtin_bit_cast(bf16x8, query(nb, kb, ch));
                         if constexpr (QR) {
                             constexpr int KCI = decltype(kcv)::value;
-                            b[nb] = bhr[4 * KCI + kb][nb];
+                            bl[nb] = __builtin_bit_cast(bf16x8, sm.u.p.qlo[wn * QW + 32 * nb + r][4 * KCI + ch]);
                         } else {
-                            b[nb] = __builtin_bit_cast(halfx8, sm.u.p.qs[buf][wn * QW + 32 * nb + r][ch]);
+                            bl[nb] = __builtin_bit_cast(bf16x8, sm.u.p.qs[buf][wn * QW + 32 * nb + r][ch + 4]);
                         }
                     }
 #pragma unroll
                     for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
                         for (int nb = 0; nb < NB; ++nb)
-                            acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                                a[mb], b[nb], (FIRST && kb == 0) ? zero : acc[mb][nb], 0, 0, 0);
+                            acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[mb], bh[nb], z ? zero : acc[mb][nb], 0, 0, 0);
+#pragma unroll
+                    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+                        for (int nb = 0; nb < NB; ++nb)
+                            acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[mb], bl[nb], acc[mb][nb], 0, 0, 0);
+#pragma unroll
+                    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+                        for (int nb = 0; nb < NB; ++nb)
+                            acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[mb], bh[nb], acc[mb][nb], 0, 0, 0);
                 }
-            } else {
-#pragma unroll
-            for (int kb = 0; kb < 2; ++kb) {
-                const int ch = 2 * kb + h; // float4 column of the high parts; +4: low parts
-                bf16x8 ah[2], al[2], bh[NB], bl[NB];
-#pragma unroll
-                for (int mb = 0; mb < 2; ++mb) {
-                    ah[mb] = __builtin_bit_cast(bf16x8, sm.u.p.xs[buf][wm * 64 + 32 * mb + r][ch]);
-                    al[mb] = __builtin_bit_cast(bf16x8, sm.u.p.xs[buf][wm * 64 + 32 * mb + r][ch + 4]);
-                }
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb) {
-                    bh[nb] = __builtin_bit_cast(bf16x8, sm.u.p.qs[buf][wn * QW + 32 * nb + r][ch]);
-                    bl[nb] = __builtin_bit_cast(bf16x8, sm.u.p.qs[buf][wn * QW + 32 * nb + r][ch + 4]);
-                }
-                const bool z = FIRST && kb == 0;
-#pragma unroll
-                for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-                    for (int nb = 0; nb < NB; ++nb)
-                        acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[mb], bh[nb], z ? zero : acc[mb][nb], 0, 0, 0);
-#pragma unroll
-                for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-                    for (int nb = 0; nb < NB; ++nb)
-                        acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah[mb], bl[nb], acc[mb][nb], 0, 0, 0);
-#pragma unroll
-                for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-                    for (int nb = 0; nb < NB; ++nb)
-                        acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al[mb], bh[nb], acc[mb][nb], 0, 0, 0);
-            }
             }
         };
         // the MFMA block at raised wave priority: the SIMD's other wave (in its epilogue's
         // VALU work) yields issue slots to it, which keeps the matrix core fed.  In the
-        // register-query layout the priority also grows with the chunk (1, 2): of
-        // two waves in their MFMA steps, the one nearer its epilogue issues first, so it
-        // reaches the epilogue while the other still has matrix work.  Their phases drift
-        // apart instead of locking (split operands, 4 chunks: cross select -1.5 to 2 %).  With restaged query
-        // panels (12 to 24 chunks a tile) a graded priority measured slower, so those
-        // steps stay at 1.
+        // register-query layout the priority also grows with the chunk (half: 1, 2; split: 1,
+        // 2, 3, 3): of two waves in their MFMA steps, the one nearer its epilogue issues
+        // first, so it reaches the epilogue while the other still has matrix work.  Their
+        // phases drift apart instead of locking (split operands: cross select -1.5 to 2 %).
+        // With restaged query panels (12 to 24 chunks a tile) a graded priority measured
+        // slower, so those steps stay at 1.
         if constexpr (QR) {
             constexpr uint32_t KCP = decltype(kcv)::value + 1u;
             __builtin_amdgcn_s_setprio(KCP > 3u ? 3 : (int16_t)KCP);
@@ -1343,6 +1374,10 @@ __global__ __launch_bounds__(select_threads<NB>(), (LT <= 8 ? 2 : 1)) void ung_s
         for (uint32_t s = 0; s < total; s += QR_NK) {
             step(s, std::integral_constant<uint32_t, 0>{});
             step(s + 1, std::integral_constant<uint32_t, 1>{});
+            if constexpr (!HALF) {
+                step(s + 2, std::integral_constant<uint32_t, 2>{});
+                step(s + 3, std::integral_constant<uint32_t, 3>{});
+            }
         }
     } else {
         for (uint32_t s = 0; s < total; ++s)

@@ -539,9 +539,9 @@ int launch_select_t(ung_hip_ctx *ctx, hipStream_t stream, const SelectParams &P,
     const int th = select_threads<NB>();
     SelectParams R = P;
     R.run_log2 = HALF && long_rows(P.dp) && n_items <= (1u << 28) ? LONG_RUN_LOG2 : XCD_RUN_NONE;
-    if constexpr (NB == 2 && HALF) {
-        // two columns per lane and half operands of 128 dimensions: the register-query layout
-        if (P.dp == (uint32_t)(QR_NK * KC) && ctx->qreg) {
+    if constexpr (NB == 2) {
+        // two columns per lane and operand rows of 128 dimensions: the register-query layout
+        if (P.dp == (uint32_t)(qr_chunks<HALF>() * KC) && ctx->qreg) {
             if (mode == LOAD_BUF32)
                 return excl ? launch_items(ctx, stream, P, n_items, mode, th, ung_select_kernel<LT, LOAD_BUF32, true, NB, true, HALF>)
                             : launch_items(ctx, stream, P, n_items, mode, th, ung_select_kernel<LT, LOAD_BUF32, false, NB, true, HALF>);
