@@ -972,6 +972,15 @@ constexpr uint32_t MAX_FALLBACK_SPLITS = 1024;
 constexpr uint32_t HALF_RETRY = 512;
 constexpr uint32_t HALF_RETRY_MIN = 256;
 
+// Operand bytes that a select streams over n items, rows of dp words.
+uint64_t select_bytes(const Item *items, uint64_t n, uint32_t dp)
+{
+    uint64_t rows = 0;
+    for (uint64_t i = 0; i < n; ++i)
+        rows += (uint64_t)items[i].q_cnt + (items[i].v_end - items[i].v_begin);
+    return rows * dp * sizeof(uint32_t);
+}
+
 int plan_finish(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, PlanMem &m, ung_hip_stats *st)
 {
     int rc;
@@ -989,6 +998,8 @@ int plan_finish(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, Pla
             st->merge_ms += b;
             st->kernel_ms += a + b;
             st->select_launches += 1;
+            st->select_bytes += select_bytes(pl.items.data(), pl.items.size(), operands_of(ctx, m.half).dp);
+            st->padded_pairs += pl.padded;
         }
         pick_operands(ctx, k, (pl.jobs[0].flags & 1u) != 0, false, m); // (its partial rows are no longer than the half ones)
         if ((rc = plan_launch_select(ctx, ws, pl, k, m)) || (rc = plan_launch_merge(ctx, ws, pl, k, m, st, false)))
@@ -1062,10 +1073,7 @@ int plan_finish(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, Pla
         st->fallback_rows += nflag;
         st->pairs += pl.pairs;
         st->padded_pairs += pl.padded;
-        uint64_t rows_streamed = 0;
-        for (const Item &it : pl.items)
-            rows_streamed += (uint64_t)it.q_cnt + (it.v_end - it.v_begin);
-        st->select_bytes += rows_streamed * operands_of(ctx, m.half).dp * sizeof(uint32_t);
+        st->select_bytes += select_bytes(pl.items.data(), pl.items.size(), operands_of(ctx, m.half).dp);
         st->rows += pl.rows;
         st->work_items += pl.items.size();
         st->select_launches += 1;
