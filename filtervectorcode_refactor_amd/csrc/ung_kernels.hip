@@ -93,6 +93,10 @@ struct SelectParams {
     uint32_t n_items; // items of this launch
     uint32_t *item_ctr; // next item to take: one counter, or one per XCD (zeroed before the launch)
     uint32_t run_log2;  // log2 of the consecutive items one XCD takes (XCD_RUN_NONE: one counter)
+    uint32_t *give_up;  // half operands: [0] rows seen that will not be certified, weighted
+                        // (uncertifiable), [1] items taken when the select gave up
+    uint32_t give_limit; // more than this in [0]: the blocks take no further items
+    float eps_coef, eps_lin, rmax; // the certificate's error bound (bound_ea), in fp32 for this estimate
     uint32_t lp;      // entries per partial row (approximate top-Lp)
     uint32_t x_bytes; // bytes of the split base set (buffer range of the 32-bit-offset kernels)
 };
@@ -475,7 +479,9 @@ __device__ __forceinline__ uint32_t take_item(uint32_t *ctr, uint32_t *slot)
 // an XCD): run j of the list belongs to XCD j % 8, whose blocks take its items through their
 // own counter; where an XCD has no item left its blocks take the other XCDs'.  A counter
 // hands out ascending positions, so one position past the list ends it, and n_items blocks
-// meet n_items positions (n_items <= 2^28: positions stay below 2^32).  Which XCD a block really runs on changes the speed alone.
+// meet n_items positions (n_items <= RUN_MAX_ITEMS: positions stay below 2^32, also past
+// give_up's step).  Which XCD a block really runs on changes the speed alone.
+constexpr uint32_t RUN_MAX_ITEMS = 1u << 26;
 constexpr uint32_t N_XCD = 8;
 constexpr uint32_t XCD_RUN_NONE = 32;
 __device__ __forceinline__ uint32_t take_item_run(uint32_t *ctr, uint32_t run_log2, uint32_t n_items, uint32_t *slot)
@@ -491,6 +497,45 @@ __device__ __forceinline__ uint32_t take_item_run(uint32_t *ctr, uint32_t run_lo
     }
     __syncthreads();
     return *slot;
+}
+
+// Half operands: a call that leaves too many rows uncertified is repeated on the split
+// operands, so its select counts the rows that the merge will not certify, and past
+// P.give_limit it gives up: the item counters step past the end of the list, no block takes a
+// further item, and the merge exits on the same count (some partial rows are unwritten).  On
+// data off the origin, against a whole half select and merge and against the split operands
+// alone: lists of 32 at 300k x 128 2.7 -> 1.05 ms (0.85), cross 1M x 128 38.5 -> 25.0 ms
+// (22.7), 78k x 100, k = 10 1.85 -> 1.4 ms (1.0), 300k x 384 13.6 -> 13.0 ms (10.5: its first
+// 512 items take as long as the rest).  Where they certify the rows: 1M x 128 select 8.45 ->
+// 8.47 ms, lists at 300k x 384 0.638 -> 0.647 ms.  Looking at the count within an item as well
+// gave 1M 24.4 and 300k x 384 12.4 ms, and cost every select 1 %.
+//
+// uncertifiable: whether the merge will leave a row uncertified, as far as its approximate
+// distances tell: dk its k-th one, A the bound of the candidates left out, qn = |q|^2, all
+// unscaled.  A partial row of one of several splits tells less (the whole row's k-th distance
+// is not known here): it counts one where an unsplit row counts GIVE_UNSPLIT, and not at all
+// with a tie at dk (more copies of one vector in this split than the row is long).  The merge
+// alone decides what is certified; this decides only how soon a call gives up.
+constexpr uint32_t GIVE_UNSPLIT = 16;
+__device__ __forceinline__ bool uncertifiable(const SelectParams &P, bool unsplit, float dk, float A, float qn)
+{
+    const float r = sqrtf(fmaxf(qn, 0.0f)) + P.rmax;
+    return dk < INFINITY && !(A - (P.eps_coef * r + P.eps_lin) * r > dk) && (unsplit || A != dk);
+}
+
+// One thread a wave adds the wave's count; the one that passes the limit steps the item
+// counters on and leaves the number of items taken so far in P.give_up[1].
+__device__ __forceinline__ void count_uncertifiable(const SelectParams &P, uint32_t n)
+{
+    if (n == 0u)
+        return;
+    const uint32_t before = atomicAdd(P.give_up, n);
+    if (before <= P.give_limit && before + n > P.give_limit) {
+        uint32_t taken = 0u;
+        for (uint32_t x = 0; x < (P.run_log2 != XCD_RUN_NONE ? N_XCD : 1u); ++x)
+            taken += atomicAdd(P.item_ctr + x, P.n_items);
+        P.give_up[1] = min(taken, P.n_items);
+    }
 }
 
 // Pre-filter bound in s-space: s = |x|^2/2 - <x,q> and a = fl(2s + |q|^2).  Returns c
@@ -1410,12 +1455,14 @@ __global__ __launch_bounds__(select_threads<NB>(), (LT <= 8 ? 2 : 1)) void ung_s
         __syncthreads();
         // one thread per query: 4-way merge of the sorted queues -> approximate top-Lp;
         // the first value left out joins the bound
+        [[maybe_unused]] bool bad = false; // (the first wave's threads hold the rows)
         if (tid < rows_here) {
             const int jl = tid;
             const uint32_t ql = (uint32_t)(pass * 64 + jl);
             const size_t prow = (size_t)jb.part_base + (size_t)it.split * jb.q_count + it.q_off + ql;
             int hp[4] = {0, 0, 0, 0};
             float drop = INFINITY;
+            [[maybe_unused]] float dk = INFINITY;
             for (uint32_t t = 0; t <= Lp; ++t) {
                 float bd = INFINITY;
                 uint32_t bi = NONE;
@@ -1438,6 +1485,8 @@ __global__ __launch_bounds__(select_threads<NB>(), (LT <= 8 ? 2 : 1)) void ung_s
                 }
                 P.part_ids[prow * Lp + t] = bi;
                 P.part_dist[prow * Lp + t] = bd * P.inv_s2;
+                if (HALF && t + 1u == P.k)
+                    dk = bd;
                 if (bl >= 0)
                     ++hp[bl];
             }
@@ -1446,6 +1495,13 @@ __global__ __launch_bounds__(select_threads<NB>(), (LT <= 8 ? 2 : 1)) void ung_s
             for (int l = 0; l < 4; ++l)
                 A = fminf(A, sm.u.r.alist[jl][l]);
             P.part_bound[prow] = A * P.inv_s2; // approximate-distance space
+            if constexpr (HALF)
+                bad = uncertifiable(P, jb.n_split == 1u, dk * P.inv_s2, A * P.inv_s2, sm.qn[ql] * P.inv_s2);
+        }
+        if constexpr (HALF) {
+            const uint32_t n_bad = (uint32_t)__popcll(__ballot(bad));
+            if (tid == 0)
+                count_uncertifiable(P, n_bad * (jb.n_split == 1u ? GIVE_UNSPLIT : 1u));
         }
     }
 }
@@ -2046,6 +2102,19 @@ __global__ __launch_bounds__(KNN_THREADS, 1) void ung_knn_select_kernel(SelectPa
         for (int i = 0; i < 16; ++i)
             next = (uint32_t)(16 * p + i) == Lp ? d[i] : next;
         next = quad_min(next);
+        if constexpr (HALF) {
+            float dk = INFINITY; // the k-th entry (k <= Lp < KNN_OUT)
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                dk = (uint32_t)(16 * p + i) + 1u == P.k ? d[i] : dk;
+            dk = quad_min(dk);
+            const bool bad =
+                p == 0 && (uint32_t)q < qcnt &&
+                uncertifiable(P, jb.n_split == 1u, dk * P.inv_s2, fminf(sm.tau[q], next) * P.inv_s2, sm.qn[q] * P.inv_s2);
+            const uint32_t n_bad = (uint32_t)__popcll(__ballot(bad));
+            if (lane == 0)
+                count_uncertifiable(P, n_bad * (jb.n_split == 1u ? GIVE_UNSPLIT : 1u));
+        }
         if ((uint32_t)q < qcnt) {
             const size_t prow = (size_t)jb.part_base + (size_t)it.split * jb.q_count + it.q_off + (uint32_t)q;
             const uint32_t id0 = P.seg_start[jb.seg_begin] + it.v_begin; // group jobs: one segment
@@ -2086,6 +2155,8 @@ struct MergeParams {
     uint32_t n_mitems;   // items of this launch
     uint32_t xcd_spread; // 1: consecutive items to one XCD (see ung_merge_kernel)
     uint32_t qlds;       // 1: the launch gave MERGE_ROWS * d floats of LDS for query rows
+    const uint32_t *give_up; // the select gave up (*give_up > give_limit): no partial rows to merge
+    uint32_t give_limit;
 };
 
 // The MI355X's XCDs; the dispatcher hands a launch's workgroups to them round-robin.
@@ -2114,9 +2185,10 @@ __global__ __launch_bounds__(64 * MERGE_ROWS) void ung_merge_kernel(MergeParams 
         if (li >= M.n_mitems)
             return; // whole block; no block barrier in this kernel
     }
+    const uint32_t gave_up = *M.give_up;
     const MergeItem mi = M.mitems[li];
-    if ((uint32_t)w >= mi.q_cnt)
-        return; // whole wave; no block barrier below
+    if (gave_up > M.give_limit || (uint32_t)w >= mi.q_cnt)
+        return; // whole wave; no block barrier below (gave up: some partial rows are unwritten)
     const Job jb = M.jobs[mi.job];
     const uint32_t ql = mi.q_off + (uint32_t)w;
     const uint32_t q = jb.q_begin + ql;

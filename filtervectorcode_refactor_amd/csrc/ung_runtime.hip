@@ -200,6 +200,12 @@ StageLayout stage_layout(const Plan &pl)
     return L;
 }
 
+// Words of a call's flag array: rows flagged for the rescan, the select's item counters (one,
+// or one per XCD), and (half operands) the rows it found uncertifiable, the items taken when it
+// gave up.
+constexpr uint32_t FLAG_ROWS = 0, FLAG_ITEMS = 1, FLAG_GIVE_UP = FLAG_ITEMS + N_XCD, FLAG_TAKEN = FLAG_GIVE_UP + 1,
+                   FLAG_WORDS = FLAG_TAKEN + 1;
+
 // Where a planned call reads its work lists, keeps its partial rows and flags, and
 // writes its result rows.
 struct PlanMem {
@@ -209,7 +215,7 @@ struct PlanMem {
     uint32_t *seg_start = nullptr, *seg_vend = nullptr;
     uint32_t *part_ids = nullptr;
     float *part_dist = nullptr, *part_bound = nullptr;
-    uint32_t *flag_count = nullptr; // [0]: rows flagged for the rescan, then the select's item counters
+    uint32_t *flag_count = nullptr; // FLAG_* words
     uint2 *flagged = nullptr;
     uint2 *tiny = nullptr;          // Plan::tiny
     uint32_t *out_ids = nullptr;    // result rows
@@ -243,7 +249,7 @@ struct Workspace {
     DevBuf<uint32_t> part_ids;
     DevBuf<float> part_dist;
     DevBuf<float> part_bound;
-    DevBuf<uint32_t> flag_count; // [0]: rows flagged for the rescan, then the select's item counters
+    DevBuf<uint32_t> flag_count; // FLAG_* words
     DevBuf<uint2> flagged;
     DevBuf<uint2> tiny;
     DevBuf<uint32_t> fb_ids; // rescan range results
@@ -538,7 +544,7 @@ int launch_select_t(ung_hip_ctx *ctx, hipStream_t stream, const SelectParams &P,
     constexpr int NB = LT <= 8 ? 2 : 1;
     const int th = select_threads<NB>();
     SelectParams R = P;
-    R.run_log2 = HALF && long_rows(P.dp) && n_items <= (1u << 28) ? LONG_RUN_LOG2 : XCD_RUN_NONE;
+    R.run_log2 = HALF && long_rows(P.dp) && n_items <= RUN_MAX_ITEMS ? LONG_RUN_LOG2 : XCD_RUN_NONE;
     if constexpr (NB == 2) {
         // two columns per lane and operand rows of 128 dimensions: the register-query layout
         if (P.dp == (uint32_t)(qr_chunks<HALF>() * KC) && ctx->qreg) {
@@ -676,7 +682,7 @@ int workspace_mem(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, R
         (rc = ws.mitems.ensure(pl.n_mitems)) || (rc = ws.seg_start.ensure(pl.seg_start.size())) ||
         (rc = ws.seg_vend.ensure(pl.seg_vend.size())) ||
         (rc = ws.part_ids.ensure(pl.part_rows * lp)) || (rc = ws.part_dist.ensure(pl.part_rows * lp)) ||
-        (rc = ws.part_bound.ensure(pl.part_rows)) || (rc = ws.flag_count.ensure(1 + N_XCD)) ||
+        (rc = ws.part_bound.ensure(pl.part_rows)) || (rc = ws.flag_count.ensure(FLAG_WORDS)) ||
         (rc = ws.flagged.ensure(std::max<uint64_t>(pl.rows, 1))) || (rc = ws.tiny.ensure(pl.n_tiny + 1)))
         return rc;
     if (!pl.jobs.empty()) {
@@ -787,6 +793,22 @@ size_t merge_qlds_bytes(uint32_t d)
     return d <= MERGE_QLDS ? (size_t)MERGE_ROWS * d * sizeof(float) : 0;
 }
 
+// A half pre-selection that leaves more than one row in HALF_RETRY uncertified (and more
+// than HALF_RETRY_MIN, below which the rescan takes less than another launch) is repeated on
+// the split operands before the rescan.  The exact rescan handles about 2.3e9 pairs/s at
+// d = 128 (cfg2: 14,060 rows of 27,400 candidates, 170 ms), the split select 1.4e12
+// (20.6e9 pairs, 14.4 ms): repeating pays from about one row in 600 on.
+constexpr uint32_t HALF_RETRY = 512;
+constexpr uint32_t HALF_RETRY_MIN = 256;
+
+// Most rows that a call's pre-selection may leave uncertified, and the count of rows found
+// uncertifiable (GIVE_UNSPLIT each) from which its select gives up.
+uint32_t retry_limit(const PlanMem &m, const Plan &pl)
+{
+    return m.half ? (uint32_t)std::max<uint64_t>(HALF_RETRY_MIN, pl.rows / HALF_RETRY) : ~0u;
+}
+uint32_t give_limit(const PlanMem &m, const Plan &pl) { return m.half ? GIVE_UNSPLIT * retry_limit(m, pl) : ~0u; }
+
 // Runs a planned job list on workspace `ws` (its stream and events) with the memory of
 // `m`; result rows already initialised by the caller when some rows have no job.
 // plan_launch uploads the work lists and enqueues the select and merge kernels;
@@ -850,7 +872,7 @@ int plan_launch(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, Pla
 int plan_launch_select(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, PlanMem &m)
 {
     int rc;
-    hipLaunchKernelGGL(ung_zero_u32_kernel, dim3(1), dim3(64), 0, ws.stream, m.flag_count, 1u + N_XCD);
+    hipLaunchKernelGGL(ung_zero_u32_kernel, dim3(1), dim3(64), 0, ws.stream, m.flag_count, FLAG_WORDS);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipEventRecord(ws.ev[0], ws.stream));
 
@@ -870,8 +892,13 @@ int plan_launch_select(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t
     P.part_ids = m.part_ids;
     P.part_dist = m.part_dist;
     P.part_bound = m.part_bound;
-    P.item_ctr = m.flag_count + 1;
+    P.item_ctr = m.flag_count + FLAG_ITEMS;
     P.run_log2 = XCD_RUN_NONE;
+    P.give_up = m.flag_count + FLAG_GIVE_UP;
+    P.give_limit = give_limit(m, pl);
+    P.eps_coef = (float)o.coef;
+    P.eps_lin = (float)o.lin;
+    P.rmax = (float)o.rmax;
     P.lp = lp;
     const uint32_t n_items = (uint32_t)pl.items.size();
     const bool excl = (pl.jobs[0].flags & 1u) != 0; // one kind of job per plan
@@ -927,8 +954,10 @@ int plan_launch_merge(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t 
     M.out_ids = m.out_ids;
     M.out_dist = m.out_dist;
     M.out_size = m.out_size;
-    M.flag_count = m.flag_count;
+    M.flag_count = m.flag_count + FLAG_ROWS;
     M.flagged = m.flagged;
+    M.give_up = m.flag_count + FLAG_GIVE_UP;
+    M.give_limit = give_limit(m, pl);
     // group kNN plans (exclusive jobs: a group against itself) of long rows spread their
     // items over the XCDs in contiguous ranges (d = 768: intra merge 11.3 -> 8.5 ms; at
     // d = 128 and 384 it measured the same or 2 % slower)
@@ -964,14 +993,6 @@ int plan_launch_merge(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t 
 constexpr uint32_t FALLBACK_RANGE = 256;
 constexpr uint32_t MAX_FALLBACK_SPLITS = 1024;
 
-// A half pre-selection that leaves more than one row in HALF_RETRY uncertified (and more
-// than HALF_RETRY_MIN, below which the rescan takes less than another launch) is repeated on
-// the split operands before the rescan.  The exact rescan handles about 2.3e9 pairs/s at
-// d = 128 (cfg2: 14,060 rows of 27,400 candidates, 170 ms), the split select 1.4e12
-// (20.6e9 pairs, 14.4 ms): repeating pays from about one row in 600 on.
-constexpr uint32_t HALF_RETRY = 512;
-constexpr uint32_t HALF_RETRY_MIN = 256;
-
 // Operand bytes that a select streams over n items, rows of dp words.
 uint64_t select_bytes(const Item *items, uint64_t n, uint32_t dp)
 {
@@ -986,10 +1007,11 @@ int plan_finish(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, Pla
     int rc;
     if (pl.jobs.empty())
         return UNG_HIP_OK;
-    uint32_t nflag = 0;
-    HIPCHECK(hipMemcpyAsync(&nflag, m.flag_count, sizeof(uint32_t), hipMemcpyDeviceToHost, ws.stream));
+    uint32_t flags[FLAG_WORDS] = {};
+    HIPCHECK(hipMemcpyAsync(flags, m.flag_count, sizeof(flags), hipMemcpyDeviceToHost, ws.stream));
     HIPCHECK(hipStreamSynchronize(ws.stream));
-    if (m.half && nflag > HALF_RETRY_MIN && (uint64_t)nflag * HALF_RETRY > pl.rows) {
+    uint32_t nflag = flags[FLAG_ROWS];
+    if (nflag > retry_limit(m, pl) || flags[FLAG_GIVE_UP] > give_limit(m, pl)) {
         if (st) {
             float a = 0, b = 0;
             HIPCHECK(hipEventElapsedTime(&a, ws.ev[0], ws.ev[1]));
@@ -998,13 +1020,18 @@ int plan_finish(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, Pla
             st->merge_ms += b;
             st->kernel_ms += a + b;
             st->select_launches += 1;
-            st->select_bytes += select_bytes(pl.items.data(), pl.items.size(), operands_of(ctx, m.half).dp);
-            st->padded_pairs += pl.padded;
+            // the items it ran: all, or those at the head of the staged list
+            const Item *items = reinterpret_cast<const Item *>(m.stage + stage_layout(pl).oi);
+            const bool gave_up = flags[FLAG_GIVE_UP] > give_limit(m, pl);
+            const uint64_t n = gave_up ? std::min<uint64_t>(flags[FLAG_TAKEN], pl.items.size()) : pl.items.size();
+            st->select_bytes += select_bytes(items, n, operands_of(ctx, m.half).dp);
+            for (uint64_t i = 0; i < n; ++i)
+                st->padded_pairs += (uint64_t)BQ * ((items[i].v_end - items[i].v_begin + BC - 1) / BC * BC);
         }
         pick_operands(ctx, k, (pl.jobs[0].flags & 1u) != 0, false, m); // (its partial rows are no longer than the half ones)
         if ((rc = plan_launch_select(ctx, ws, pl, k, m)) || (rc = plan_launch_merge(ctx, ws, pl, k, m, st, false)))
             return rc;
-        HIPCHECK(hipMemcpyAsync(&nflag, m.flag_count, sizeof(uint32_t), hipMemcpyDeviceToHost, ws.stream));
+        HIPCHECK(hipMemcpyAsync(&nflag, m.flag_count + FLAG_ROWS, sizeof(uint32_t), hipMemcpyDeviceToHost, ws.stream));
         HIPCHECK(hipStreamSynchronize(ws.stream));
     }
     if (nflag > 0) {
@@ -1023,7 +1050,7 @@ int plan_finish(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, Pla
         F.jobs = m.jobs;
         F.seg_start = m.seg_start;
         F.seg_vend = m.seg_vend;
-        F.flag_count = m.flag_count;
+        F.flag_count = m.flag_count + FLAG_ROWS;
         F.flagged = m.flagged;
         F.splits = S;
         F.out_ids = m.out_ids;
@@ -2074,7 +2101,7 @@ int scratch_mem(ung_hip_ctx *ctx, const Plan &pl, uint32_t lp, PlanMem &m)
     const uint64_t o_pid = take(pl.part_rows * lp * sizeof(uint32_t));
     const uint64_t o_pd = take(pl.part_rows * lp * sizeof(float));
     const uint64_t o_pb = take(pl.part_rows * sizeof(float));
-    const uint64_t o_fc = take((1 + N_XCD) * sizeof(uint32_t));
+    const uint64_t o_fc = take(FLAG_WORDS * sizeof(uint32_t));
     const uint64_t o_fl = take(std::max<uint64_t>(pl.rows, 1) * sizeof(uint2));
     const uint64_t o_tiny = take((pl.n_tiny + 1) * sizeof(uint2));
     if (off > UNG_HIP_NOALLOC_SCRATCH_BYTES) {

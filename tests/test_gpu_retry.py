@@ -2,7 +2,8 @@
 the operands' rounding error grows with the vectors' norms, their distances do not).  Such a
 call is repeated on the split operands.  Every entry point, the register-query layout and the
 restaged panels; rows bit for bit against the CPU oracle, or against a context that has the
-split operands alone; the statistics count both selects."""
+split operands alone; the statistics count both selects.  The half select gives up soon: past
+a count of rows it knows it will not certify it runs no further item, and no merge."""
 import os
 
 import numpy as np
@@ -123,3 +124,53 @@ def test_noalloc_split_rows_only(ctx, split_ctx):
     wi, wd, ws, st2 = split_ctx.cross_topk(gb, op, oi, 6)
     assert st["select_launches"] == 1 and st["select_bytes"] == st2["select_bytes"]
     _assert_rows_equal(ids, dist, size, wi, wd, ws, "noalloc on split rows")
+
+
+def _check_cross_gives_up(ctx, split_ctx, X, gb, op, oi, k, what):
+    ctx.prepare_vectors(X)
+    split_ctx.prepare_vectors(X)
+    ids, dist, size, st = ctx.cross_topk(gb, op, oi, k)
+    wi, wd, ws, st2 = split_ctx.cross_topk(gb, op, oi, k)
+    _assert_rows_equal(ids, dist, size, wi, wd, ws, what)
+    assert st["select_launches"] == 2 and st2["select_launches"] == 1
+    # the items in flight when it gives up (at most 512 blocks), of 2,000 or 900
+    assert st2["padded_pairs"] < st["padded_pairs"] < 1.6 * st2["padded_pairs"]
+    assert st["select_bytes"] > st2["select_bytes"]
+
+
+@pytest.mark.parametrize("d,k", [(100, 6), (200, 6), (128, 12), (200, 32)])
+def test_cross_gives_up(ctx, split_ctx, d, k):
+    print(f"give up cross d={d} k={k}", flush=True)
+    sizes = [64] * 2000 + [1000]
+    gb = np.concatenate([[0, 0], np.cumsum(sizes)]).astype(np.uint32)
+    op = np.minimum(np.maximum(np.arange(2003) - 1, 0), 2000).astype(np.uint32)
+    oi = np.full(2000, 2001, np.uint32)
+    X = _far(int(gb[-1]), d, 20 if k == 6 else 12, 0.1, d + k)
+    _check_cross_gives_up(ctx, split_ctx, X, gb, op, oi, k, f"d={d} k={k}")
+
+
+def test_cross_gives_up_on_split_rows(ctx, split_ctx):
+    """300 unions of 70,000 candidates, three splits each."""
+    print("give up split rows", flush=True)
+    sizes = [128] * 300 + [70_000]
+    gb = np.concatenate([[0, 0], np.cumsum(sizes)]).astype(np.uint32)
+    op = np.minimum(np.maximum(np.arange(303) - 1, 0), 300).astype(np.uint32)
+    X = _far(int(gb[-1]), 128, 12, 0.1, 9)
+    _check_cross_gives_up(ctx, split_ctx, X, gb, op, np.full(300, 301, np.uint32), 12, "split rows")
+
+
+@pytest.mark.parametrize("d,k", [(64, 32), (128, 32), (200, 32), (200, 63)])
+def test_lists_give_up(ctx, split_ctx, d, k):
+    """2,100 items of 300-point groups: the filter-and-buffer select (d <= 128) and the register
+    queues."""
+    print(f"give up lists d={d} k={k}", flush=True)
+    size = np.full(700, 300, np.uint32)
+    begin = np.arange(700, dtype=np.uint32) * 300
+    X = _far(210_000, d, 12, 0.1, d)
+    ctx.prepare_vectors(X)
+    split_ctx.prepare_vectors(X)
+    ids, dist, st = ctx.group_knn(begin, size, k)
+    wi, wd, st2 = split_ctx.group_knn(begin, size, k)
+    _assert_rows_equal(ids, dist, None, wi, wd, None, f"lists d={d} k={k}")
+    assert st["select_launches"] == 2 and st2["select_launches"] == 1
+    assert st["padded_pairs"] < 1.6 * st2["padded_pairs"]
