@@ -4,14 +4,15 @@ call is repeated on the split operands.  Every entry point, the register-query l
 restaged panels; rows bit for bit against the CPU oracle, or against a context that has the
 split operands alone; the statistics count both selects.  The half select gives up soon: past
 a count of rows it knows it will not certify it runs no further item, and no merge."""
+import ctypes as C
 import os
 
 import numpy as np
 import pytest
-import torch
 
 import filtervectorcode_refactor_amd as F
 from test_gpu_parity import _assert_rows_equal
+from test_zz_no_alloc import DeviceRows
 
 pytestmark = pytest.mark.gpu
 
@@ -93,12 +94,12 @@ def test_overlapped_calls(ctx, oracle, d, norm, k):
 
 
 def _noalloc(ctx, n, k, *graph):
-    out = (torch.empty(n, k, dtype=torch.int32, device="cuda"), torch.empty(n, k, device="cuda"),
-           torch.empty(n, dtype=torch.int32, device="cuda"))
-    torch.cuda.synchronize()
-    st = ctx.cross_topk_noalloc(*graph, k, *[t.data_ptr() for t in out])
-    ids, dist, size = [t.cpu().numpy() for t in out]
-    return ids.view(np.uint32), dist, size, st
+    rows = DeviceRows(C.CDLL("libamdhip64.so"), n, k)
+    try:
+        st = ctx.cross_topk_noalloc(*graph, k, *rows.addrs())
+        return *rows.download(), st
+    finally:
+        rows.free()
 
 
 @pytest.mark.parametrize("d,norm,k", [(128, 30, 6), (128, 30, 40), (512, 45, 12)])
