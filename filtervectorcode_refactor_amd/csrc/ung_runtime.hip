@@ -59,11 +59,19 @@ struct AllocCount {
     AllocCount &operator=(const AllocCount &) = delete;
 };
 
+// A failed allocation leaves no error behind for the launch checks of later calls.
 hipError_t counted_malloc(void **p, size_t bytes)
 {
     ++t_alloc_calls;
-    return hipMalloc(p, bytes);
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess)
+        (void)hipGetLastError();
+    return e;
 }
+
+// A buffer of the call on this thread could not grow (with_memory); test hook: none can.
+thread_local bool t_short = false;
+thread_local bool t_refuse_growth = false;
 
 template <class T>
 struct DevBuf {
@@ -78,9 +86,10 @@ struct DevBuf {
         p = nullptr;
         cap = 0;
         size_t want = n + n / 4 + 64;
-        hipError_t e = counted_malloc((void **)&p, want * sizeof(T));
+        hipError_t e = t_refuse_growth ? hipErrorOutOfMemory : counted_malloc((void **)&p, want * sizeof(T));
         if (e != hipSuccess) {
             p = nullptr;
+            t_short = true;
             set_error("hipMalloc(%zu bytes) failed: %s", want * sizeof(T), hipGetErrorString(e));
             return UNG_HIP_EDEVICE;
         }
@@ -349,6 +358,9 @@ struct ung_hip_ctx {
     bool qreg = true;
     // test hook: UNG_HIP_NO_HALF=1 at create keeps every pre-selection on the split operands
     bool half = true;
+    // test hook: UNG_HIP_SHORT_WITH_HALF=1 at create lets no buffer grow while the half base set
+    // is allocated (with_memory)
+    bool short_with_half = false;
     // test hook: UNG_HIP_EPS_SCALE=s (s >= 1) at create widens the certification error
     // bound by s, which sends more rows (all, for a huge s) through the exact rescan
     double eps_scale = 1.0;
@@ -1084,6 +1096,7 @@ int plan_finish(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, Pla
     HIPCHECK(hipEventRecord(ws.ev[3], ws.stream));
     HIPCHECK(hipEventSynchronize(ws.ev[3]));
     if (m.rescanned) {
+        m.rescanned->clear();
         for (const uint2 &f : flagged_host)
             m.rescanned->push_back(pl.jobs[f.x].out_row + f.y);
         std::sort(m.rescanned->begin(), m.rescanned->end());
@@ -1362,6 +1375,36 @@ void drain_after_failure(ung_hip_ctx *ctx)
     }
 }
 
+// Frees the half base set: the split operands serve every call without it.  (hp, half_s2 and
+// half_res stay: a list call in flight that used it still accounts with them.)
+void drop_half(ung_hip_ctx *ctx)
+{
+    drain_after_failure(ctx); // selects in flight read it
+    (void)hipFree(ctx->XH);
+    ctx->XH = nullptr;
+    ctx->half_ok = false;
+}
+
+// Runs a call; where a buffer could not grow for want of device memory, the half base set
+// makes room and the call runs once more, its rows shorter and its plan unsplit: a base set
+// that leaves little memory gets the results that it got without the half set.
+template <class F>
+int with_memory(ung_hip_ctx *ctx, ung_hip_stats *st, F &&call)
+{
+    const ung_hip_stats before = st ? *st : ung_hip_stats{};
+    t_short = false;
+    t_refuse_growth = ctx && ctx->short_with_half && ctx->XH;
+    int rc = call();
+    t_refuse_growth = false;
+    if (rc == UNG_HIP_OK || !t_short || !ctx || !ctx->XH)
+        return rc;
+    drop_half(ctx);
+    clear_error();
+    if (st)
+        *st = before;
+    return call();
+}
+
 // Result rows of a cross call, initialised (padding) on the first workspace's stream.
 int cross_prepare_result(ung_hip_ctx *ctx, uint32_t k)
 {
@@ -1489,8 +1532,11 @@ int intra_end(ung_hip_ctx *ctx, ung_hip_stats *st)
         return rc;
     ctx->intra_pending = false;
     const uint32_t list_k = ctx->intra_list_k;
-    if ((rc = plan_finish(ctx, ctx->ws[1], ctx->intra_plan, list_k, ctx->intra_mem, &ctx->intra_stats)) ||
-        (rc = group_complete(ctx, ctx->ws[1], ctx->intra_plan, list_k))) {
+    rc = with_memory(ctx, &ctx->intra_stats, [&] {
+        int r = plan_finish(ctx, ctx->ws[1], ctx->intra_plan, list_k, ctx->intra_mem, &ctx->intra_stats);
+        return r ? r : group_complete(ctx, ctx->ws[1], ctx->intra_plan, list_k);
+    });
+    if (rc) {
         drain_after_failure(ctx);
         return rc;
     }
@@ -1973,9 +2019,8 @@ int prepare_common(ung_hip_ctx *ctx, const float *src, bool src_device, uint64_t
     // workspaces: a base set that fits without it is served by the split operands.
     size_t mem_free = 0, mem_total = 0;
     HIPCHECK(hipMemGetInfo(&mem_free, &mem_total));
-    if (N * hp * sizeof(uint32_t) + mem_total / 8 <= mem_free &&
+    if (ctx->half && N * hp * sizeof(uint32_t) + mem_total / 8 <= mem_free &&
         counted_malloc((void **)&ctx->XH, N * hp * sizeof(uint32_t)) != hipSuccess) {
-        (void)hipGetLastError();
         ctx->XH = nullptr;
     }
     HIPCHECK(hipMemcpyAsync(ctx->X, src, N * dim * sizeof(float),
@@ -2021,6 +2066,10 @@ int prepare_common(ung_hip_ctx *ctx, const float *src, bool src_device, uint64_t
     ctx->hp = hp;
     ctx->half_res = std::sqrt((double)res2) * (1.0 + 1e-6);
     ctx->half_ok = ctx->half && ctx->XH && e >= HALF_EMIN && e <= HALF_EMAX && ctx->half_res <= ctx->rmax * 0x1p-10;
+    if (ctx->XH && !ctx->half_ok) { // nothing will read it
+        (void)hipFree(ctx->XH);
+        ctx->XH = nullptr;
+    }
     if (ctx->half_ok) {
         const uint32_t sb = half_scale_bits(e);
         float scale;
@@ -2262,6 +2311,8 @@ int ung_hip_create(int device, ung_hip_ctx **out)
         ctx->qreg = s[0] != '1';
     if (const char *s = std::getenv("UNG_HIP_NO_HALF"))
         ctx->half = s[0] != '1';
+    if (const char *s = std::getenv("UNG_HIP_SHORT_WITH_HALF"))
+        ctx->short_with_half = s[0] == '1';
     if (const char *s = std::getenv("UNG_HIP_NO_KNN"))
         ctx->knn = s[0] != '1';
     if (const char *s = std::getenv("UNG_HIP_PRUNE_EXACT"); s && s[0] == '1')
@@ -2434,7 +2485,7 @@ int ung_hip_cross_topk_device(ung_hip_ctx *ctx, uint32_t G, const uint32_t *grou
 {
     clear_error();
     AllocCount alloc_count(st);
-    return cross_device(ctx, G, group_begin, out_ptr, out_idx, k, st);
+    return with_memory(ctx, st, [&] { return cross_device(ctx, G, group_begin, out_ptr, out_idx, k, st); });
 }
 
 int ung_hip_cross_topk(ung_hip_ctx *ctx, uint32_t G, const uint32_t *group_begin, const uint32_t *out_ptr,
@@ -2448,7 +2499,7 @@ int ung_hip_cross_topk(ung_hip_ctx *ctx, uint32_t G, const uint32_t *group_begin
         return UNG_HIP_EINVAL;
     }
     const auto t0 = clk::now();
-    int rc = cross_device(ctx, G, group_begin, out_ptr, out_idx, k, st);
+    int rc = with_memory(ctx, st, [&] { return cross_device(ctx, G, group_begin, out_ptr, out_idx, k, st); });
     if (rc)
         return rc;
     rc = download(ctx, ctx->cross, out_ids, out_dist, out_size, st);
@@ -2498,8 +2549,10 @@ int ung_hip_additional_edges(ung_hip_ctx *ctx, uint32_t G, const uint32_t *group
 {
     clear_error();
     AllocCount alloc_count(st);
-    return additional_device(ctx, G, group_begin, out_ptr, out_idx, num_cross, edge_ptr, edge_from, edge_to, capacity,
-                             n_edges, st);
+    return with_memory(ctx, st, [&] {
+        return additional_device(ctx, G, group_begin, out_ptr, out_idx, num_cross, edge_ptr, edge_from, edge_to,
+                                 capacity, n_edges, st);
+    });
 }
 
 int ung_hip_group_knn_device(ung_hip_ctx *ctx, uint32_t n_groups, const uint32_t *grp_begin,
@@ -2507,7 +2560,7 @@ int ung_hip_group_knn_device(ung_hip_ctx *ctx, uint32_t n_groups, const uint32_t
 {
     clear_error();
     AllocCount alloc_count(st);
-    return group_device(ctx, n_groups, grp_begin, grp_size, list_k, st);
+    return with_memory(ctx, st, [&] { return group_device(ctx, n_groups, grp_begin, grp_size, list_k, st); });
 }
 
 int ung_hip_group_knn(ung_hip_ctx *ctx, uint32_t n_groups, const uint32_t *grp_begin, const uint32_t *grp_size,
@@ -2520,7 +2573,7 @@ int ung_hip_group_knn(ung_hip_ctx *ctx, uint32_t n_groups, const uint32_t *grp_b
         return UNG_HIP_EINVAL;
     }
     const auto t0 = clk::now();
-    int rc = group_device(ctx, n_groups, grp_begin, grp_size, list_k, st);
+    int rc = with_memory(ctx, st, [&] { return group_device(ctx, n_groups, grp_begin, grp_size, list_k, st); });
     if (rc)
         return rc;
     rc = download(ctx, ctx->group, out_ids, out_dist, nullptr, st);
@@ -2535,7 +2588,9 @@ int ung_hip_cross_intra_begin(ung_hip_ctx *ctx, uint32_t G, const uint32_t *grou
 {
     clear_error();
     AllocCount alloc_count(st);
-    return cross_intra_begin(ctx, G, group_begin, out_ptr, out_idx, k, n_groups, grp_begin, grp_size, list_k, st);
+    return with_memory(ctx, st, [&] {
+        return cross_intra_begin(ctx, G, group_begin, out_ptr, out_idx, k, n_groups, grp_begin, grp_size, list_k, st);
+    });
 }
 
 int ung_hip_intra_end(ung_hip_ctx *ctx, ung_hip_stats *st)
@@ -2616,12 +2671,10 @@ int ung_hip_download_group(ung_hip_ctx *ctx, uint32_t *out_ids, float *out_dist,
     return download(ctx, ctx->group, out_ids, out_dist, nullptr, st);
 }
 
-int ung_hip_pack_anchor_rows(ung_hip_ctx *ctx, uint32_t tagore_k, uint32_t final_degree, uint32_t head_keep,
-                             uint32_t anchor_tail, uint32_t anchor_slots, uint32_t bidir_anchor,
-                             uint32_t *out_graph, uint32_t *entry_points, ung_hip_stats *st)
+static int pack_anchor_rows(ung_hip_ctx *ctx, uint32_t tagore_k, uint32_t final_degree, uint32_t head_keep,
+                            uint32_t anchor_tail, uint32_t anchor_slots, uint32_t bidir_anchor,
+                            uint32_t *out_graph, uint32_t *entry_points, ung_hip_stats *st)
 {
-    clear_error();
-    AllocCount alloc_count(st);
     if (!ctx || !ctx->group.valid) {
         set_error("ung_hip_pack_anchor_rows: run ung_hip_group_knn(_device) first");
         return UNG_HIP_ESTATE;
@@ -2688,11 +2741,21 @@ int ung_hip_pack_anchor_rows(ung_hip_ctx *ctx, uint32_t tagore_k, uint32_t final
     return UNG_HIP_OK;
 }
 
-int ung_hip_prune_group_graph(ung_hip_ctx *ctx, uint32_t forward_cap, uint32_t reverse_cap, uint32_t final_degree,
-                              float alpha, uint32_t *out_graph, uint32_t *entry_points, ung_hip_stats *st)
+int ung_hip_pack_anchor_rows(ung_hip_ctx *ctx, uint32_t tagore_k, uint32_t final_degree, uint32_t head_keep,
+                             uint32_t anchor_tail, uint32_t anchor_slots, uint32_t bidir_anchor,
+                             uint32_t *out_graph, uint32_t *entry_points, ung_hip_stats *st)
 {
     clear_error();
     AllocCount alloc_count(st);
+    return with_memory(ctx, st, [&] {
+        return pack_anchor_rows(ctx, tagore_k, final_degree, head_keep, anchor_tail, anchor_slots, bidir_anchor,
+                                out_graph, entry_points, st);
+    });
+}
+
+static int prune_group_graph(ung_hip_ctx *ctx, uint32_t forward_cap, uint32_t reverse_cap, uint32_t final_degree,
+                             float alpha, uint32_t *out_graph, uint32_t *entry_points, ung_hip_stats *st)
+{
     if (!ctx || !ctx->group.valid) {
         set_error("ung_hip_prune_group_graph: run ung_hip_group_knn(_device) first");
         return UNG_HIP_ESTATE;
@@ -2789,6 +2852,16 @@ int ung_hip_prune_group_graph(ung_hip_ctx *ctx, uint32_t forward_cap, uint32_t r
         st->rows += rows;
     }
     return UNG_HIP_OK;
+}
+
+int ung_hip_prune_group_graph(ung_hip_ctx *ctx, uint32_t forward_cap, uint32_t reverse_cap, uint32_t final_degree,
+                              float alpha, uint32_t *out_graph, uint32_t *entry_points, ung_hip_stats *st)
+{
+    clear_error();
+    AllocCount alloc_count(st);
+    return with_memory(ctx, st, [&] {
+        return prune_group_graph(ctx, forward_cap, reverse_cap, final_degree, alpha, out_graph, entry_points, st);
+    });
 }
 
 int ung_hip_synchronize(ung_hip_ctx *ctx)
