@@ -148,6 +148,7 @@ struct Plan {
     uint64_t padded = 0;
     uint64_t rows = 0;
     uint64_t max_item_cand = 0;    // largest candidate range of an item
+    bool fine = false;             // cross plan of fine splits (fine_splits)
     // jobs of a few queries and a small union (tiny_job), scanned exactly without the
     // select and the merge (n_split = 0): [0].x = n_tiny, then (job, 0) for each
     ung::RawVector<uint2> tiny;
@@ -392,32 +393,76 @@ uint32_t split_size(uint64_t u)
 
 // Half operand rows (hp words) so long that the query panels of an XCD's 64 resident blocks,
 // re-read for every candidate tile, take several times its 4 MB L2 (16 KB panels at d = 64;
-// from d = 449 on, 8 MB and more).  Such a select is bound by what it fetches past the L2
-// (2M x 768: 7.4 TB/s), so the blocks of one XCD take runs of 64 consecutive items
-// (take_item_run) and the cross plan's runs are all splits of a few query blocks.
-// Measured at both sides: 2M x 768 select 76.6 -> 71.2 ms (runs alone 75.0), lists of 10
-// groups at 400k x 768 4.73 -> 4.37 ms (runs of 32: 4.74); 1M x 384 8.05 -> 8.60 ms, whose
-// operands mostly hit the L2 (20 GB fetched) and whose few long items a run puts on one XCD.
+// from d = 449 on, 8 MB and more).  Two rules make such a select share panels and candidates
+// in the L2:
 bool long_rows(uint32_t hp) { return (uint64_t)hp * sizeof(uint32_t) * BQ * 64u >= (8ull << 20); }
-constexpr uint32_t LONG_RUN_LOG2 = 6;
 
-// Candidates per split of a cross job of u candidates with long rows: up to 4 splits of at
-// least 2048 candidates (16 tiles).  8 splits: select 69.7 ms, but merge 5.1 -> 6.9 ms.
-constexpr uint64_t FINE_SPLITS = 4, FINE_SPLIT_MIN = 2048;
-uint32_t split_size_cross(uint64_t u, bool fine)
+// fine splits: the unions of a cross plan are cut into up to 4 splits of at least 2048
+// candidates (16 tiles), their items in query-major order,
+//  * where the longest of the coarse items takes two thirds of the select's time or more
+//    (the tiles a resident block has to do), so that few long items would leave the chip
+//    idle at the end.  Call coarse -> 4 splits: 100k x 768, k = 6 2.9 -> 1.4 ms; 190k x 512,
+//    k = 6 4.3 -> 2.2; 100k x 512, k = 10 2.4 -> 1.4, k = 32 2.8 -> 2.05; 240k x 512 (0.75 of the
+//    time), k = 10 5.2 -> 4.2, k = 32 the same; 300k x 512 (0.54), k = 32 7.7 -> 8.2;
+//  * otherwise with queues of 8 (two blocks a CU), which share panels and candidates in the L2
+//    better so, no more splits than the merge sorts in one wave (64 entries: 4 at k <= 6, 3 at
+//    k = 7 and 8).  k = 6: 400k x 449 3.24 -> 3.12 ms, 400k x 512 7.6 -> 6.6, 400k x 768 4.46 ->
+//    4.27, 800k x 768 14.0 -> 13.8; 3 against 4 splits at k = 8: 400k x 512 6.9, 7.1, 2M x 768
+//    80.2, 80.6.  With one block a CU (k >= 9) they lose: 400k x 768 k = 10 6.2 -> 6.5 ms, k = 32
+//    9.75 -> 10.5, 2M x 768 k = 32 126.8 -> 132.9.
+// 8 splits: 2M x 768 select 71.2 -> 69.7 ms, merge 5.1 -> 6.9.  Up to 8M rows: three more
+// partial rows are at most 3.6 GB there for an even plan (18 entries), 16 GB for an uneven one
+// (80); a call without room for them is planned coarse (with_memory).
+constexpr uint32_t FINE_SPLITS = 4;
+constexpr uint64_t FINE_SPLIT_MIN = 2048;
+constexpr uint64_t N_CU = 256;
+uint32_t pick_lp(uint32_t k, int lt, uint32_t margin);
+uint32_t lp_margin(uint32_t k, uint32_t d, bool half);
+int pick_lt(uint32_t k);
+bool may_split_fine(const ung_hip_ctx *ctx)
+{
+    return ctx->half_ok && long_rows(ctx->hp) && ctx->N <= (1ull << 23);
+}
+// Whether a plan whose coarse items have `tiles` tiles in all, the longest `longest`, is uneven.
+bool uneven_plan(uint32_t k, uint64_t tiles, uint64_t longest)
+{
+    return 2 * tiles < 3 * longest * (pick_lt(k) == 8 ? 2 * N_CU : N_CU); // (resident blocks)
+}
+// Splits of an even plan (0: coarse).
+uint32_t even_splits(const ung_hip_ctx *ctx, uint32_t k)
+{
+    const int lt = pick_lt(k);
+    return lt == 8 ? std::min<uint32_t>(FINE_SPLITS, 64u / pick_lp(k, lt, lp_margin(k, ctx->d, true))) : 0;
+}
+
+// Candidates per split of a cross job of u candidates.
+uint32_t split_size_cross(uint64_t u, uint32_t fine)
 {
     const uint32_t coarse = split_size(u);
     if (!fine)
         return coarse;
-    const uint64_t ns = std::min<uint64_t>(FINE_SPLITS, std::max<uint64_t>(1, u / FINE_SPLIT_MIN));
+    const uint64_t ns = std::min<uint64_t>(fine, std::max<uint64_t>(1, u / FINE_SPLIT_MIN));
     return (uint32_t)std::min<uint64_t>(coarse, ((u + ns - 1) / ns + BC - 1) / BC * BC);
 }
 
-// Fine splits only up to 8M rows: at most 4 splits x 80 entries x 8 bytes a row of partial
-// rows (16 entries at k = 6), which larger base sets may not have to spare.
-bool fine_splits(const ung_hip_ctx *ctx)
+// runs: the blocks of one XCD take runs of 64 consecutive items (take_item_run), of a finely
+// split cross plan all splits of a few query blocks, of a group plan the query blocks of one
+// group.  Only for plans that give every XCD many runs, or items so long that their sharing
+// outweighs the uneven ends: finely split plans of 8192 items, group plans of more than 4096
+// candidates an item on average.  Call one counter -> runs: cross 2M x 768 82.0 -> 77.1 ms, 2M
+// x 512 53.5 -> 52.2, 800k x 768 13.75 -> 13.55 (11k items), but 400k x 512 6.34 -> 6.5 (6.4k
+// items), 30k x 768 0.816 -> 0.849; groups above 4096 points 400k x 512 5.47 -> 5.06, 400k x
+// 768 7.49 -> 7.08, 1M x 768 the same, but lists of 128 to 4096 points 400k x 768 2.75 -> 2.82
+// and 100k x 768 0.86 -> 1.16.
+constexpr uint32_t LONG_RUN_LOG2 = 6;
+constexpr uint64_t RUN_MIN_ITEMS = 8192, RUN_MIN_CAND = 4096;
+uint32_t item_runs(const Plan &pl, uint32_t hp, bool group)
 {
-    return ctx->half_ok && long_rows(ctx->hp) && ctx->N <= (1ull << 23);
+    const uint64_t n = pl.items.size();
+    if (!long_rows(hp) || n > RUN_MAX_ITEMS)
+        return XCD_RUN_NONE;
+    const bool runs = group ? pl.padded > n * BQ * RUN_MIN_CAND : pl.fine && n >= RUN_MIN_ITEMS;
+    return runs ? LONG_RUN_LOG2 : XCD_RUN_NONE;
 }
 
 // Empties a plan, keeping the capacity of its lists.
@@ -430,6 +475,7 @@ void plan_reset(Plan &pl)
     pl.seg_vend.clear();
     pl.n_mitems = 0;
     pl.max_item_cand = 0;
+    pl.fine = false;
     pl.tiny.clear();
     pl.n_tiny = 0;
     pl.part_lp = 0;
@@ -555,8 +601,6 @@ int launch_select_t(ung_hip_ctx *ctx, hipStream_t stream, const SelectParams &P,
     // queues longer than 8 take the one-column-per-lane layout (two waves per SIMD)
     constexpr int NB = LT <= 8 ? 2 : 1;
     const int th = select_threads<NB>();
-    SelectParams R = P;
-    R.run_log2 = HALF && long_rows(P.dp) && n_items <= RUN_MAX_ITEMS ? LONG_RUN_LOG2 : XCD_RUN_NONE;
     if constexpr (NB == 2) {
         // two columns per lane and operand rows of 128 dimensions: the register-query layout
         if (P.dp == (uint32_t)(qr_chunks<HALF>() * KC) && ctx->qreg) {
@@ -568,10 +612,10 @@ int launch_select_t(ung_hip_ctx *ctx, hipStream_t stream, const SelectParams &P,
         }
     }
     if (mode == LOAD_BUF32)
-        return excl ? launch_items(ctx, stream, R, n_items, mode, th, ung_select_kernel<LT, LOAD_BUF32, true, NB, false, HALF>)
-                    : launch_items(ctx, stream, R, n_items, mode, th, ung_select_kernel<LT, LOAD_BUF32, false, NB, false, HALF>);
-    return excl ? launch_items(ctx, stream, R, n_items, mode, th, ung_select_kernel<LT, LOAD_WIDE, true, NB, false, HALF>)
-                : launch_items(ctx, stream, R, n_items, mode, th, ung_select_kernel<LT, LOAD_WIDE, false, NB, false, HALF>);
+        return excl ? launch_items(ctx, stream, P, n_items, mode, th, ung_select_kernel<LT, LOAD_BUF32, true, NB, false, HALF>)
+                    : launch_items(ctx, stream, P, n_items, mode, th, ung_select_kernel<LT, LOAD_BUF32, false, NB, false, HALF>);
+    return excl ? launch_items(ctx, stream, P, n_items, mode, th, ung_select_kernel<LT, LOAD_WIDE, true, NB, false, HALF>)
+                : launch_items(ctx, stream, P, n_items, mode, th, ung_select_kernel<LT, LOAD_WIDE, false, NB, false, HALF>);
 }
 
 template <bool HALF>
@@ -905,7 +949,7 @@ int plan_launch_select(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t
     P.part_dist = m.part_dist;
     P.part_bound = m.part_bound;
     P.item_ctr = m.flag_count + FLAG_ITEMS;
-    P.run_log2 = XCD_RUN_NONE;
+    P.run_log2 = m.half ? item_runs(pl, o.dp, (pl.jobs[0].flags & 1u) != 0) : XCD_RUN_NONE;
     P.give_up = m.flag_count + FLAG_GIVE_UP;
     P.give_limit = give_limit(m, pl);
     P.eps_coef = (float)o.coef;
@@ -1157,7 +1201,9 @@ int check_ready(ung_hip_ctx *ctx)
 // validates its groups; after a prefix over the chunks pass 2 writes them at its offsets.
 struct PlanChunk {
     uint32_t g_begin = 0, g_end = 0; // groups [g_begin, g_end)
-    uint64_t jobs = 0, segs = 0, items = 0, mitems = 0, part_rows = 0, pairs = 0, padded = 0, rows = 0, tiny = 0;
+    uint64_t jobs = 0, segs = 0, mitems = 0, pairs = 0, rows = 0, tiny = 0, longest = 0;
+    // by number of splits: coarse, those of an even plan, those of an uneven one
+    uint64_t items[3] = {}, part_rows[3] = {}, padded[3] = {};
     int rc = UNG_HIP_OK;
     char msg[192] = {};
 };
@@ -1166,7 +1212,7 @@ struct PlanChunk {
 // (the out-groups' ranges in LNG row order), and its items (query blocks x splits,
 // split-major).  Two passes over chunks of groups on the context's worker pool.
 int build_cross_plan(ung_hip_ctx *ctx, uint32_t G, const uint32_t *group_begin, const uint32_t *out_ptr,
-                     const uint32_t *out_idx, Plan &pl, bool fine)
+                     const uint32_t *out_idx, Plan &pl, uint32_t fine_k)
 {
     if (!group_begin || !out_ptr || (out_ptr[G + 1] > 0 && !out_idx)) {
         set_error("ung_hip_cross_topk: null group_begin/out_ptr/out_idx");
@@ -1210,6 +1256,9 @@ int build_cross_plan(ung_hip_ctx *ctx, uint32_t G, const uint32_t *group_begin, 
         std::snprintf((c).msg, sizeof((c).msg), __VA_ARGS__);                              \
         return;                                                                            \
     } while (0)
+    const bool may_fine = fine_k > 0 && may_split_fine(ctx);
+    const uint32_t fine_of[3] = {0u, may_fine ? even_splits(ctx, fine_k) : 0u, FINE_SPLITS};
+    const uint32_t n_fine = may_fine ? 3u : 1u;
     auto pass1 = [&](int64_t t) {
         PlanChunk &c = ch[t];
         for (uint32_t g = c.g_begin; g < c.g_end; ++g) {
@@ -1243,12 +1292,17 @@ int build_cross_plan(ung_hip_ctx *ctx, uint32_t G, const uint32_t *group_begin, 
                 c.tiny += 1;
                 continue;
             }
-            const uint64_t sv = split_size_cross(u, fine), ns = (u + sv - 1) / sv, qb = (qn + BQ - 1) / BQ;
-            c.items += ns * qb;
             c.mitems += (qn + MERGE_ROWS - 1) / MERGE_ROWS;
-            c.part_rows += (uint64_t)qn * ns;
-            const uint64_t last = u - (ns - 1) * sv;
-            c.padded += (uint64_t)BQ * qb * ((ns - 1) * sv + (last + BC - 1) / BC * BC);
+            const uint64_t qb = (qn + BQ - 1) / BQ;
+            for (uint32_t f = 0; f < n_fine; ++f) {
+                const uint64_t sv = split_size_cross(u, fine_of[f]), ns = (u + sv - 1) / sv;
+                c.items[f] += ns * qb;
+                c.part_rows[f] += qn * ns;
+                const uint64_t last = u - (ns - 1) * sv;
+                c.padded[f] += (uint64_t)BQ * qb * ((ns - 1) * sv + (last + BC - 1) / BC * BC);
+                if (f == 0)
+                    c.longest = std::max<uint64_t>(c.longest, (std::min(sv, u) + BC - 1) / BC);
+            }
         }
     };
 #undef PLAN_FAIL
@@ -1256,6 +1310,16 @@ int build_cross_plan(ung_hip_ctx *ctx, uint32_t G, const uint32_t *group_begin, 
         pass1(0);
     else
         ctx->pool->run(nch, pass1);
+    uint32_t way = 0;
+    if (may_fine) {
+        uint64_t padded = 0, longest = 0;
+        for (const PlanChunk &c : ch) {
+            padded += c.padded[0];
+            longest = std::max(longest, c.longest);
+        }
+        way = uneven_plan(fine_k, padded / ((uint64_t)BQ * BC), longest) ? 2 : 1;
+    }
+    const uint32_t fine = fine_of[way];
     uint64_t n_jobs = 0, n_segs = 0, n_items = 0;
     std::vector<uint64_t> o_job(nch), o_seg(nch), o_item(nch), o_part(nch), o_tiny(nch);
     for (uint32_t t = 0; t < nch; ++t) {
@@ -1271,17 +1335,18 @@ int build_cross_plan(ung_hip_ctx *ctx, uint32_t G, const uint32_t *group_begin, 
         pl.n_tiny += ch[t].tiny;
         n_jobs += ch[t].jobs;
         n_segs += ch[t].segs;
-        n_items += ch[t].items;
-        pl.part_rows += ch[t].part_rows;
+        n_items += ch[t].items[way];
+        pl.part_rows += ch[t].part_rows[way];
         pl.n_mitems += ch[t].mitems;
         pl.pairs += ch[t].pairs;
-        pl.padded += ch[t].padded;
+        pl.padded += ch[t].padded[way];
         pl.rows += ch[t].rows;
     }
     if (pl.part_rows >= 0xFFFFFFFFull || n_segs >= 0xFFFFFFFFull) {
         set_error("ung_hip_cross_topk: partial rows exceed 2^32");
         return UNG_HIP_EINVAL;
     }
+    pl.fine = fine != 0;
     pl.jobs.resize(n_jobs);
     pl.items.resize(n_items);
     pl.seg_start.resize(n_segs);
@@ -1440,7 +1505,7 @@ int cross_device(ung_hip_ctx *ctx, uint32_t G, const uint32_t *group_begin, cons
     const auto t0 = clk::now();
     Plan &pl = ctx->plan0;
     plan_reset(pl);
-    if ((rc = build_cross_plan(ctx, G, group_begin, out_ptr, out_idx, pl, fine_splits(ctx))))
+    if ((rc = build_cross_plan(ctx, G, group_begin, out_ptr, out_idx, pl, k)))
         return rc;
     if (st)
         st->plan_ms += ms_since(t0);
@@ -1474,7 +1539,7 @@ int cross_intra_begin(ung_hip_ctx *ctx, uint32_t G, const uint32_t *group_begin,
     const auto t0 = clk::now();
     Plan &pl = ctx->plan0;
     plan_reset(pl);
-    if ((rc = build_cross_plan(ctx, G, group_begin, out_ptr, out_idx, pl, fine_splits(ctx))))
+    if ((rc = build_cross_plan(ctx, G, group_begin, out_ptr, out_idx, pl, k)))
         return rc;
     if (st)
         st->plan_ms += ms_since(t0);
@@ -2237,7 +2302,7 @@ int cross_noalloc(ung_hip_ctx *ctx, uint32_t G, const uint32_t *group_begin, con
     ctx->cross.rescanned.clear();
     Plan &pl = ctx->plan0;
     plan_reset(pl);
-    if ((rc = build_cross_plan(ctx, G, group_begin, out_ptr, out_idx, pl, false))) // (no more scratch than it has to)
+    if ((rc = build_cross_plan(ctx, G, group_begin, out_ptr, out_idx, pl, 0))) // (no more scratch than it has to)
         return rc;
     if (st)
         st->plan_ms += ms_since(t0);
