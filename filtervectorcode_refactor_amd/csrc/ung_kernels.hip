@@ -76,8 +76,8 @@ typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 struct SelectParams {
-    const uint32_t *xs; // pre-selection operands: [N][dp] words, the half base set (ung_half_kernel)
-                        // or the split base set (ung_split_kernel)
+    const uint32_t *xs; // pre-selection operands: [N][dp] words, the half or the split base set
+                        // (ung_operands_kernel)
     const float *xn;
     uint32_t dp;        // words per operand row, whole chunks of KC words
     float s2, inv_s2;   // squared scale of the operands (a power of two; 1 for the split set) and
@@ -2779,70 +2779,65 @@ __global__ __launch_bounds__(64) void ung_fallback_merge_kernel(FallbackParams F
 // small kernels
 // ---------------------------------------------------------------------------
 
-// Split base set for the MFMA pre-selection: x = hi + lo + r with hi = bf16(x) and
-// lo = bf16(x - hi) (x - hi is exact: both lie within a factor 2 of each other), so
-// |r| <= 2^-18 |x|.  Row n holds dp words (dp = d rounded up to a multiple of KC); its
-// chunk c (dimensions 32c .. 32c+31) is 16 words of hi pairs then 16 words of lo pairs,
-// dimension 32c+2j in the low half of word j.  Dimensions >= d are zero.
-__global__ __launch_bounds__(256) void ung_split_kernel(const float *__restrict__ X, uint64_t N, uint32_t d,
-                                                        uint32_t dp, uint32_t *__restrict__ XS)
+// Blocks of the upload's kernels: eight a CU fill it, and more only queue at the maxima's
+// words (an atomic each, about 12 ns: 8192 blocks took 96 us over 50k x 64, whose rows are
+// read in 5).
+constexpr uint32_t UPLOAD_BLOCKS = 2048;
+constexpr int NORM_ROWS = 4, OPERAND_ROWS = 2; // rows a wave has in flight
+
+// The largest of `v` over the block's four waves into *to (w: four words of LDS): most blocks
+// find a larger value there and leave it.
+__device__ __forceinline__ void block_max(unsigned int v, unsigned int *w, unsigned int *to)
 {
-    const uint64_t per_row = dp / 2; // one (hi word, lo word) pair per thread
-    const uint64_t total = N * per_row;
-    for (uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total;
-         t += (uint64_t)gridDim.x * blockDim.x) {
-        const uint64_t n = t / per_row;
-        const uint32_t w = (uint32_t)(t - n * per_row); // pair index within the row
-        const uint32_t c = w >> 4, j = w & 15u;
-        const uint32_t dim = 32u * c + 2u * j;
-        const float *x = X + n * d;
-        const float x0 = dim < d ? x[dim] : 0.0f;
-        const float x1 = dim + 1 < d ? x[dim + 1] : 0.0f;
-        const uint32_t h0 = bf16_rne(x0), h1 = bf16_rne(x1);
-        const uint32_t l0 = bf16_rne(x0 - __uint_as_float(h0 << 16));
-        const uint32_t l1 = bf16_rne(x1 - __uint_as_float(h1 << 16));
-        uint32_t *row = XS + n * dp + 32u * c;
-        row[j] = h0 | (h1 << 16);
-        row[16 + j] = l0 | (l1 << 16);
+    if ((threadIdx.x & 63) == 0)
+        w[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const unsigned int m = max(max(w[0], w[1]), max(w[2], w[3]));
+        if (m > __hip_atomic_load(to, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            atomicMax(to, m);
     }
 }
 
-// Squared norms (one wave per row, grid-stride over rows; lanes stride the row), the
-// largest of them (maxbits[0]) and the largest |coordinate| (maxbits[1]): block-wide maxima,
-// then one atomic per block.  Accumulated in fp64 and rounded once, so each cached norm is
-// within 2^-24 (relative) of |x|^2.  Non-negative floats order as their bit patterns (a NaN
-// or infinite coordinate gives an exponent of 255).
+// Squared norms (one wave per row, NORM_ROWS rows at a time; lanes stride the row), the
+// largest of them (maxbits[0]) and the largest |coordinate| (maxbits[1]).  Accumulated in fp64
+// and rounded once, so each cached norm is within 2^-24 (relative) of |x|^2.  Non-negative
+// floats order as their bit patterns (a NaN or infinite coordinate gives an exponent of 255).
 __global__ __launch_bounds__(256) void ung_norm_kernel(const float *__restrict__ X, uint64_t N, uint32_t d,
                                                        float *__restrict__ xn, unsigned int *__restrict__ maxbits)
 {
     __shared__ unsigned int wmax[2][4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint64_t nwaves = (uint64_t)gridDim.x * 4u;
+    const uint64_t step = (uint64_t)gridDim.x * 4u * NORM_ROWS;
     unsigned int mx = 0u, am = 0u;
-    for (uint64_t row = (uint64_t)blockIdx.x * 4u + (uint64_t)wave; row < N; row += nwaves) {
-        const float *x = X + row * d;
-        double sd = 0.0;
+    for (uint64_t row = ((uint64_t)blockIdx.x * 4u + (uint64_t)wave) * NORM_ROWS; row < N; row += step) {
+        const int rows = (int)min((uint64_t)NORM_ROWS, N - row);
+        double sd[NORM_ROWS] = {};
         for (uint32_t t = lane; t < d; t += 64) {
-            sd = __builtin_fma((double)x[t], (double)x[t], sd);
-            am = max(am, __float_as_uint(x[t]) & 0x7FFFFFFFu);
+            float v[NORM_ROWS];
+#pragma unroll
+            for (int i = 0; i < NORM_ROWS; ++i)
+                v[i] = X[(row + (uint64_t)min(i, rows - 1)) * d + t];
+#pragma unroll
+            for (int i = 0; i < NORM_ROWS; ++i) {
+                sd[i] = __builtin_fma((double)v[i], (double)v[i], sd[i]);
+                am = max(am, __float_as_uint(v[i]) & 0x7FFFFFFFu);
+            }
         }
-        for (int off = 32; off > 0; off >>= 1)
-            sd += __shfl_xor(sd, off);
-        const float s = (float)sd;
-        if (lane == 0)
-            xn[row] = s;
-        mx = max(mx, __float_as_uint(s));
+#pragma unroll
+        for (int i = 0; i < NORM_ROWS; ++i) {
+            for (int off = 32; off > 0; off >>= 1)
+                sd[i] += __shfl_xor(sd[i], off);
+            const float s = (float)sd[i];
+            if (lane == 0 && i < rows)
+                xn[row + (uint64_t)i] = s;
+            mx = max(mx, __float_as_uint(s)); // (a row past the end repeats the last one)
+        }
     }
     for (int off = 32; off > 0; off >>= 1)
         am = max(am, (unsigned int)__shfl_xor((int)am, off));
-    if (lane == 0) {
-        wmax[0][wave] = mx;
-        wmax[1][wave] = am;
-    }
-    __syncthreads();
-    if (threadIdx.x < 2)
-        atomicMax(maxbits + threadIdx.x, max(max(wmax[threadIdx.x][0], wmax[threadIdx.x][1]),
-                                             max(wmax[threadIdx.x][2], wmax[threadIdx.x][3])));
+    block_max(mx, wmax[0], maxbits);
+    block_max(am, wmax[1], maxbits + 1);
 }
 
 // Power of two that takes the largest |coordinate| (exponent field e of its bits) into
@@ -2852,49 +2847,78 @@ __global__ __launch_bounds__(256) void ung_norm_kernel(const float *__restrict__
 constexpr uint32_t HALF_EMIN = 127u - 40u, HALF_EMAX = 127u + 40u;
 __host__ __device__ inline uint32_t half_scale_bits(uint32_t e) { return (127u + 14u + 127u - e) << 23; }
 
-// The half base set: row n holds the d coordinates times the scale, rounded to fp16
-// (nearest even; below the fp16 normal range: 0), zeros up to hp words.  maxbits[2] gets
-// the largest squared norm (fp64 rounded up to fp32) of what the rounding left out of a
-// row, in the coordinates' own scale: the certificate's error term.  One wave per row.
-__global__ __launch_bounds__(256) void ung_half_kernel(const float *__restrict__ X, uint64_t N, uint32_t d,
-                                                       uint32_t hp, uint32_t *__restrict__ XH,
-                                                       unsigned int *__restrict__ maxbits)
+// The operands of the MFMA pre-selection, both sets from one pass over X; one wave per row.
+// Split base set: x = hi + lo + r with hi = bf16(x) and lo = bf16(x - hi) (x - hi is exact:
+// both lie within a factor 2 of each other), so |r| <= 2^-18 |x|.  Row n holds dp words (dp = d
+// rounded up to a multiple of KC); its chunk c (dimensions 32c .. 32c+31) is 16 words of hi
+// pairs then 16 words of lo pairs, dimension 32c+2j in the low half of word j.  Dimensions >= d
+// are zero.
+// Half base set (XH given and the largest coordinate in range): row n holds the d coordinates
+// times the scale, rounded to fp16 (nearest even; below the fp16 normal range: 0), zeros up to
+// hp words.  maxbits[2] gets the largest squared norm (fp64 rounded up to fp32) of what the
+// rounding left out of a row, in the coordinates' own scale: the certificate's error term.
+// Bound by its traffic, 4 bytes a coordinate read and 6 written: 1M x 128 282 us, 4.5 TB/s (a
+// pass for each set 204 + 211 us; 50k x 64 15 us against 7 + 96).
+__global__ __launch_bounds__(256) void ung_operands_kernel(const float *__restrict__ X, uint64_t N, uint32_t d,
+                                                           uint32_t dp, uint32_t *__restrict__ XS, uint32_t hp,
+                                                           uint32_t *__restrict__ XH,
+                                                           unsigned int *__restrict__ maxbits)
 {
     __shared__ unsigned int wmax[4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint32_t e = maxbits[1] >> 23;
-    if (e < HALF_EMIN || e > HALF_EMAX)
-        return; // (the host applies the same rule and does not use XH)
-    const float scale = __uint_as_float(half_scale_bits(e));
+    const bool half = XH && e >= HALF_EMIN && e <= HALF_EMAX; // (the host applies the same rule)
+    const float scale = half ? __uint_as_float(half_scale_bits(e)) : 1.0f;
     const float inv = 1.0f / scale; // exact
-    const uint64_t nwaves = (uint64_t)gridDim.x * 4u;
+    const uint32_t pairs = max(dp / 2u, half ? hp : 0u);
+    const uint64_t step = (uint64_t)gridDim.x * 4u * OPERAND_ROWS;
     unsigned int mx = 0u;
-    for (uint64_t row = (uint64_t)blockIdx.x * 4u + (uint64_t)wave; row < N; row += nwaves) {
-        const float *x = X + row * d;
-        double rd = 0.0;
-        for (uint32_t w = (uint32_t)lane; w < hp; w += 64u) {
-            uint32_t bits = 0u;
+    for (uint64_t row = ((uint64_t)blockIdx.x * 4u + (uint64_t)wave) * OPERAND_ROWS; row < N; row += step) {
+        const int rows = (int)min((uint64_t)OPERAND_ROWS, N - row);
+        double rd[OPERAND_ROWS] = {};
+        for (uint32_t w = (uint32_t)lane; w < pairs; w += 64u) {
+            float v[OPERAND_ROWS][2];
 #pragma unroll
-            for (uint32_t j = 0; j < 2; ++j) {
-                const uint32_t dim = 2u * w + j;
-                const float v = dim < d ? x[dim] : 0.0f;
-                const float sv = v * scale;
-                const _Float16 hv = fabsf(sv) < 0x1p-14f ? (_Float16)0.0f : (_Float16)sv;
-                const float rv = v - (float)hv * inv; // exact
-                rd = __builtin_fma((double)rv, (double)rv, rd);
-                bits |= (uint32_t)__builtin_bit_cast(uint16_t, hv) << (16u * j);
+            for (int i = 0; i < OPERAND_ROWS; ++i)
+#pragma unroll
+                for (uint32_t j = 0; j < 2; ++j)
+                    v[i][j] = 2u * w + j < d ? X[(row + (uint64_t)min(i, rows - 1)) * d + 2u * w + j] : 0.0f;
+#pragma unroll
+            for (int i = 0; i < OPERAND_ROWS; ++i) {
+                if (i < rows && 2u * w < dp) {
+                    const uint32_t h0 = bf16_rne(v[i][0]), h1 = bf16_rne(v[i][1]);
+                    const uint32_t l0 = bf16_rne(v[i][0] - __uint_as_float(h0 << 16));
+                    const uint32_t l1 = bf16_rne(v[i][1] - __uint_as_float(h1 << 16));
+                    uint32_t *out = XS + (row + (uint64_t)i) * dp + 32u * (w >> 4) + (w & 15u);
+                    out[0] = h0 | (h1 << 16);
+                    out[16] = l0 | (l1 << 16);
+                }
+                if (half) {
+                    uint32_t bits = 0u;
+#pragma unroll
+                    for (uint32_t j = 0; j < 2; ++j) {
+                        const float sv = v[i][j] * scale;
+                        const _Float16 hv = fabsf(sv) < 0x1p-14f ? (_Float16)0.0f : (_Float16)sv;
+                        const float rv = v[i][j] - (float)hv * inv; // exact
+                        rd[i] = __builtin_fma((double)rv, (double)rv, rd[i]);
+                        bits |= (uint32_t)__builtin_bit_cast(uint16_t, hv) << (16u * j);
+                    }
+                    if (i < rows)
+                        XH[(row + (uint64_t)i) * hp + w] = bits;
+                }
             }
-            XH[row * hp + w] = bits;
         }
-        for (int off = 32; off > 0; off >>= 1)
-            rd += __shfl_xor(rd, off);
-        mx = max(mx, __float_as_uint(__double2float_ru(rd)));
+        if (half) {
+#pragma unroll
+            for (int i = 0; i < OPERAND_ROWS; ++i) {
+                for (int off = 32; off > 0; off >>= 1)
+                    rd[i] += __shfl_xor(rd[i], off);
+                mx = max(mx, __float_as_uint(__double2float_ru(rd[i])));
+            }
+        }
     }
-    if (lane == 0)
-        wmax[wave] = mx;
-    __syncthreads();
-    if (threadIdx.x == 0)
-        atomicMax(maxbits + 2, max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3])));
+    if (half) // uniform
+        block_max(mx, wmax, maxbits + 2);
 }
 
 __global__ void ung_fill_rows_kernel(uint32_t *ids, float *dist, int32_t *size, uint64_t rows,

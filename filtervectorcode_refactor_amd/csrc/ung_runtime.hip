@@ -289,7 +289,7 @@ struct ung_hip_ctx {
     int device = 0;
     hipStream_t stream = nullptr; // the first workspace's stream
     hipEvent_t ev[8] = {};
-    // resident base set
+    // resident base set (X's allocation holds XS, xn and maxbits as well)
     float *X = nullptr;
     uint32_t *XS = nullptr; // split base set (bf16 hi/lo pairs) for the MFMA pre-selection
     uint32_t dp = 0;        // its row pitch in words
@@ -2076,18 +2076,29 @@ int prepare_common(ung_hip_ctx *ctx, const float *src, bool src_device, uint64_t
     const auto t0 = clk::now();
     const uint32_t dp = (dim + KC - 1) / KC * KC;
     const uint32_t hp = (dim + 2 * KC - 1) / (2 * KC) * KC; // two fp16 coordinates a word
-    HIPCHECK(counted_malloc((void **)&ctx->X, N * dim * sizeof(float)));
-    HIPCHECK(counted_malloc((void **)&ctx->XS, N * dp * sizeof(uint32_t)));
-    HIPCHECK(counted_malloc((void **)&ctx->xn, N * sizeof(float)));
-    HIPCHECK(counted_malloc((void **)&ctx->maxbits, 3 * sizeof(unsigned int)));
+    // one allocation of the coordinates, the split set, the norms and the maxima (each costs
+    // an upload and a release, those of large buffers a tenth of a millisecond), the half set
+    // in one that can go by itself
+    auto al = [](uint64_t bytes) { return (bytes + 255) & ~(uint64_t)255; };
+    const uint64_t o_xs = al(N * dim * sizeof(float)), o_xn = o_xs + al(N * dp * sizeof(uint32_t)),
+                   o_max = o_xn + al(N * sizeof(float));
+    HIPCHECK(counted_malloc((void **)&ctx->X, o_max + 3 * sizeof(unsigned int)));
+    char *const base = reinterpret_cast<char *>(ctx->X);
+    ctx->XS = reinterpret_cast<uint32_t *>(base + o_xs);
+    ctx->xn = reinterpret_cast<float *>(base + o_xn);
+    ctx->maxbits = reinterpret_cast<unsigned int *>(base + o_max);
     // The half set only where it leaves an eighth of the device memory for results and
-    // workspaces: a base set that fits without it is served by the split operands.
-    size_t mem_free = 0, mem_total = 0;
-    HIPCHECK(hipMemGetInfo(&mem_free, &mem_total));
-    if (ctx->half && N * hp * sizeof(uint32_t) + mem_total / 8 <= mem_free &&
-        counted_malloc((void **)&ctx->XH, N * hp * sizeof(uint32_t)) != hipSuccess) {
-        ctx->XH = nullptr;
+    // workspaces: a base set that fits without it is served by the split operands.  (Sets below
+    // 256 MB are not worth the query, a tenth of a 10k x 128 upload: with_memory drops them.)
+    const size_t half_bytes = N * hp * sizeof(uint32_t);
+    bool room = ctx->half;
+    if (room && half_bytes >= (256ull << 20)) {
+        size_t mem_free = 0, mem_total = 0;
+        HIPCHECK(hipMemGetInfo(&mem_free, &mem_total));
+        room = half_bytes + mem_total / 8 <= mem_free;
     }
+    if (room && counted_malloc((void **)&ctx->XH, half_bytes) != hipSuccess)
+        ctx->XH = nullptr;
     HIPCHECK(hipMemcpyAsync(ctx->X, src, N * dim * sizeof(float),
                             src_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, ctx->stream));
     hipLaunchKernelGGL(ung_zero_u32_kernel, dim3(1), dim3(64), 0, ctx->stream, (uint32_t *)ctx->maxbits, 3u);
@@ -2095,19 +2106,13 @@ int prepare_common(ung_hip_ctx *ctx, const float *src, bool src_device, uint64_t
     HIPCHECK(hipStreamSynchronize(ctx->stream));
     const double h2d = ms_since(t0);
     HIPCHECK(hipEventRecord(ctx->ev[4], ctx->stream));
-    const uint64_t norm_blocks = std::min<uint64_t>((N + 3) / 4, 8192);
-    hipLaunchKernelGGL(ung_norm_kernel, dim3((unsigned)norm_blocks), dim3(256), 0, ctx->stream, ctx->X, N, dim,
+    auto blocks = [N](uint64_t rows) { return dim3((unsigned)std::min<uint64_t>((N + rows - 1) / rows, UPLOAD_BLOCKS)); };
+    hipLaunchKernelGGL(ung_norm_kernel, blocks(4 * NORM_ROWS), dim3(256), 0, ctx->stream, ctx->X, N, dim,
                        ctx->xn, ctx->maxbits);
     HIPCHECK(hipGetLastError());
-    const uint64_t split_blocks = std::min<uint64_t>((N * (dp / 2) + 255) / 256, 16384);
-    hipLaunchKernelGGL(ung_split_kernel, dim3((unsigned)split_blocks), dim3(256), 0, ctx->stream, ctx->X, N, dim, dp,
-                       ctx->XS);
+    hipLaunchKernelGGL(ung_operands_kernel, blocks(4 * OPERAND_ROWS), dim3(256), 0, ctx->stream, ctx->X, N, dim, dp,
+                       ctx->XS, hp, ctx->XH, ctx->maxbits);
     HIPCHECK(hipGetLastError());
-    if (ctx->XH) {
-        hipLaunchKernelGGL(ung_half_kernel, dim3((unsigned)norm_blocks), dim3(256), 0, ctx->stream, ctx->X, N, dim, hp,
-                           ctx->XH, ctx->maxbits);
-        HIPCHECK(hipGetLastError());
-    }
     HIPCHECK(hipEventRecord(ctx->ev[5], ctx->stream));
     unsigned int mb[3] = {};
     HIPCHECK(hipMemcpyAsync(mb, ctx->maxbits, sizeof(mb), hipMemcpyDeviceToHost, ctx->stream));
@@ -2125,7 +2130,7 @@ int prepare_common(ung_hip_ctx *ctx, const float *src, bool src_device, uint64_t
     // max norm, inflated for the rounding of the norm cache
     ctx->rmax = std::sqrt((double)mxf * (1.0 + 1e-5)) * (1.0 + 1e-6);
     // The half operands serve the pre-selection of base sets whose largest coordinate is in
-    // ung_half_kernel's range (a zero, infinite or NaN one is not) and whose rounding error
+    // ung_operands_kernel's range (a zero, infinite or NaN one is not) and whose rounding error
     // is what fp16 gives (at most 2^-11 of a row's norm, below 2^-10 of the largest).
     const uint32_t e = mb[1] >> 23;
     ctx->hp = hp;
@@ -2446,14 +2451,8 @@ int ung_hip_release_vectors(ung_hip_ctx *ctx)
         (void)hipStreamSynchronize(ctx->stream);
     if (ctx->X)
         (void)hipFree(ctx->X);
-    if (ctx->XS)
-        (void)hipFree(ctx->XS);
     if (ctx->XH)
         (void)hipFree(ctx->XH);
-    if (ctx->xn)
-        (void)hipFree(ctx->xn);
-    if (ctx->maxbits)
-        (void)hipFree(ctx->maxbits);
     ctx->X = nullptr;
     ctx->XS = nullptr;
     ctx->dp = 0;
