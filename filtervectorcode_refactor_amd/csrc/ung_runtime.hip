@@ -236,6 +236,7 @@ struct PlanMem {
     // pre-selection of the call: half operands (one fp16 product) or split ones (three bf16
     // products), and its entries per partial row
     bool half = false;
+    bool retry = false; // repeated on the split operands where the half ones do not serve
     uint32_t lp = 0;
     // rescan range partials: grown in the workspace on demand, or a fixed region
     bool fb_grow = true;
@@ -359,6 +360,9 @@ struct ung_hip_ctx {
     bool qreg = true;
     // test hook: UNG_HIP_NO_HALF=1 at create keeps every pre-selection on the split operands
     bool half = true;
+    // test hook: UNG_HIP_NO_RETRY=1 at create rescans every row that the half operands leave
+    // uncertified instead of repeating the call, so that their partial rows can be looked at
+    bool retry = true;
     // test hook: UNG_HIP_SHORT_WITH_HALF=1 at create lets no buffer grow while the half base set
     // is allocated (with_memory)
     bool short_with_half = false;
@@ -724,6 +728,7 @@ void pick_operands(const ung_hip_ctx *ctx, uint32_t k, bool group, bool half, Pl
 {
     const uint32_t split_margin = lp_margin(k, ctx->d, false);
     m.half = half && ctx->half_ok && (!group || split_margin >= 8u);
+    m.retry = m.half && ctx->retry;
     m.lp = pick_lp(k, pick_lt(k), m.half && !group ? lp_margin(k, ctx->d, true) : split_margin);
 }
 
@@ -861,9 +866,9 @@ constexpr uint32_t HALF_RETRY_MIN = 256;
 // uncertifiable (GIVE_UNSPLIT each) from which its select gives up.
 uint32_t retry_limit(const PlanMem &m, const Plan &pl)
 {
-    return m.half ? (uint32_t)std::max<uint64_t>(HALF_RETRY_MIN, pl.rows / HALF_RETRY) : ~0u;
+    return m.retry ? (uint32_t)std::max<uint64_t>(HALF_RETRY_MIN, pl.rows / HALF_RETRY) : ~0u;
 }
-uint32_t give_limit(const PlanMem &m, const Plan &pl) { return m.half ? GIVE_UNSPLIT * retry_limit(m, pl) : ~0u; }
+uint32_t give_limit(const PlanMem &m, const Plan &pl) { return m.retry ? GIVE_UNSPLIT * retry_limit(m, pl) : ~0u; }
 
 // Runs a planned job list on workspace `ws` (its stream and events) with the memory of
 // `m`; result rows already initialised by the caller when some rows have no job.
@@ -2381,6 +2386,8 @@ int ung_hip_create(int device, ung_hip_ctx **out)
         ctx->qreg = s[0] != '1';
     if (const char *s = std::getenv("UNG_HIP_NO_HALF"))
         ctx->half = s[0] != '1';
+    if (const char *s = std::getenv("UNG_HIP_NO_RETRY"))
+        ctx->retry = s[0] != '1';
     if (const char *s = std::getenv("UNG_HIP_SHORT_WITH_HALF"))
         ctx->short_with_half = s[0] == '1';
     if (const char *s = std::getenv("UNG_HIP_NO_KNN"))
@@ -3037,6 +3044,30 @@ int ung_hip_debug_partial_rows(ung_hip_ctx *ctx, uint64_t capacity, uint32_t *qu
             }
         }
     }
+    return UNG_HIP_OK;
+}
+
+int ung_hip_debug_error_bound(ung_hip_ctx *ctx, double *coef, double *lin, double *rmax, int *half)
+{
+    clear_error();
+    if (!ctx) {
+        set_error("ung_hip_debug_error_bound: null context");
+        return UNG_HIP_EINVAL;
+    }
+    const Plan &pl = ctx->plan0;
+    if (pl.part_lp == 0) {
+        set_error("ung_hip_debug_error_bound: no partial rows of a cross or synchronous group call on the device");
+        return UNG_HIP_ESTATE;
+    }
+    const Operands o = operands_of(ctx, pl.part_half);
+    if (coef)
+        *coef = o.coef;
+    if (lin)
+        *lin = o.lin;
+    if (rmax)
+        *rmax = o.rmax;
+    if (half)
+        *half = pl.part_half ? 1 : 0;
     return UNG_HIP_OK;
 }
 

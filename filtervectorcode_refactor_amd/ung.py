@@ -280,6 +280,14 @@ class HipContext:
                                                   C.byref(ec), C.byref(rm)))
         return q, c, a, ec.value, rm.value
 
+    def debug_error_bound(self):
+        """(coef, lin, rmax, half) of the same call's certificate: |a - D| <= coef * r^2 + lin * r
+        with r = |q| + rmax, and whether its operands were the fp16 ones
+        (ung_hip_debug_error_bound; diagnostic)."""
+        coef, lin, rm, half = C.c_double(), C.c_double(), C.c_double(), C.c_int()
+        check(self.lib.ung_hip_debug_error_bound(self.h, C.byref(coef), C.byref(lin), C.byref(rm), C.byref(half)))
+        return coef.value, lin.value, rm.value, bool(half.value)
+
     def debug_partial_bounds(self):
         """(query ids, split candidate ranges [begin, end) as global ids, bounds) of the same
         call's partial rows (ung_hip_debug_partial_bounds; diagnostic)."""

@@ -285,6 +285,13 @@ int ung_hip_selftest_mfma(ung_hip_ctx *ctx, double *max_abs_err);
 int ung_hip_debug_partial_rows(ung_hip_ctx *ctx, uint64_t capacity, uint32_t *query, uint32_t *cand, float *approx,
                                uint64_t *n_entries, double *eps_coef, double *rmax);
 
+/* Diagnostic, no counterpart in the reference: the error bound the same call's rows were
+ * certified with, its two terms separately: |a - D| <= *coef * r^2 + *lin * r with
+ * r = |q| + *rmax (the eps_coef above folds both into one factor on r^2, up to twice as
+ * wide in the second), and whether its operands were the fp16 ones (*half = 1) or the
+ * split-bf16 ones (0; a call repeated on them included).  UNG_HIP_ESTATE as above. */
+int ung_hip_debug_error_bound(ung_hip_ctx *ctx, double *coef, double *lin, double *rmax, int *half);
+
 /* Diagnostic, no counterpart in the reference: the bound of every partial row of the same
  * call (the select's contract: every candidate of the row's split that the row does not
  * hold has an approximate distance a >= bound, so an exact distance D >= bound -

@@ -1,11 +1,14 @@
 """The certificate's error model checked on the hardware: every candidate a select kernel
-kept in a partial row carries its approximate squared distance a (split-bf16 MFMA,
-expansion form |q|^2 + |x|^2 - 2<q,x>), and the merge certifies rows with
-|a - D| <= eps_coef * (|q| + R)^2 for the exact squared distance D.  Here a comes back
+kept in a partial row carries its approximate squared distance a (fp16 or split-bf16
+MFMA, expansion form |q|^2 + |x|^2 - 2<q,x>), and the merge certifies rows with
+|a - D| <= eps = coef * r^2 + lin * r, r = |q| + R, for the exact squared distance D (the
+linear term is the fp16 rounding of the operands, 0 for the split ones).  Here a comes back
 through ung_hip_debug_partial_rows and D is computed in fp64 from the fp32 inputs, for
 every entry, on data chosen for cancellation (tight clusters far from the origin), mixed
-coordinate magnitudes, integer ties and three dimensions (the register-query layout at
-d = 128 and the restaged panels at 384 and 768).
+coordinate magnitudes, integer ties, data that fp16 holds exactly (no rounding term: the
+accumulation of the products alone) and three dimensions (the register-query layout at
+d = 128 and the restaged panels at 384 and 768); each on the half operands (also where a
+call would be repeated: UNG_HIP_NO_RETRY) and on the split ones (UNG_HIP_NO_HALF).
 
 The group kNN calls' selects are checked the same way, and so is the other half of the
 partial-row contract: every candidate of a row's split that the row does not hold has
@@ -13,6 +16,8 @@ a >= the row's bound (ung_hip_debug_partial_bounds), so its exact distance is at
 bound - eps.  That is the filter-and-buffer select's pre-filter and threshold at
 d <= 128 (ung_knn_select_kernel) and the register-queue select with self-exclusion at
 d = 384."""
+import os
+
 import numpy as np
 import pytest
 
@@ -22,11 +27,27 @@ from filtervectorcode_refactor_amd import datasets as D
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(scope="module")
-def ctx():
-    c = F.HipContext(0)
+@pytest.fixture(scope="module", params=["half", "split"])
+def ctx(request):
+    name = {"half": "UNG_HIP_NO_RETRY", "split": "UNG_HIP_NO_HALF"}[request.param]
+    os.environ[name] = "1"
+    try:
+        c = F.HipContext(0)
+    finally:
+        del os.environ[name]
+    c.operands = request.param
     yield c
     c.close()
+
+
+def _eps(ctx, qnorm, operands=None):
+    """The certificate's bound for rows of these norms; the call's operands must be the context's
+    (or the given ones)."""
+    coef, lin, rmax, half = ctx.debug_error_bound()
+    assert half == ((operands or ctx.operands) == "half")
+    assert half or lin == 0.0
+    r = qnorm + rmax
+    return coef * r * r + lin * r
 
 
 def _say(msg):
@@ -49,7 +70,7 @@ def _random_lng(rng, sizes):
 def _check_bound(ctx, X, gb, op, oi, label):
     ctx.prepare_vectors(X)
     _, _, _, st = ctx.cross_topk(gb, op, oi, 6)
-    q, c, a, eps_coef, rmax = ctx.debug_partial_rows()
+    q, c, a, _, rmax = ctx.debug_partial_rows()
     assert q.size > 0, f"{label}: no partial-row entries"
     Xd = X.astype(np.float64)
     # the kernel's per-query term: |q| from the cached fp32 |q|^2 (fp64 sum rounded once)
@@ -60,15 +81,15 @@ def _check_bound(ctx, X, gb, op, oi, label):
     for s in range(0, q.size, 200_000):
         qs, cs = q[s:s + 200_000].astype(np.int64), c[s:s + 200_000].astype(np.int64)
         dexact = ((Xd[qs] - Xd[cs]) ** 2).sum(axis=1)
-        eps = eps_coef * (np.sqrt(qn32[qs] * (1.0 + 1e-6)) + rmax) ** 2
+        eps = _eps(ctx, np.sqrt(qn32[qs] * (1.0 + 1e-6)))
         r = np.abs(a[s:s + 200_000].astype(np.float64) - dexact) / eps
         ratios.append(r)
         i = int(np.argmax(r))
         if r[i] > worst:
             worst, worst_i = float(r[i]), s + i
     ratios = np.concatenate(ratios)
-    _say(f"{label}: {q.size} entries, rescanned rows {st['fallback_rows']}, |a - D| / eps max {worst:.3g}, "
-         f"99.9 % {np.quantile(ratios, 0.999):.3g}, median {np.median(ratios):.3g}")
+    _say(f"{label} ({ctx.operands}): {q.size} entries, rescanned rows {st['fallback_rows']}, "
+         f"|a - D| / eps max {worst:.3g}, 99.9 % {np.quantile(ratios, 0.999):.3g}, median {np.median(ratios):.3g}")
     assert worst <= 1.0, (f"{label}: entry {worst_i} (query {q[worst_i]}, candidate {c[worst_i]}) has "
                           f"|a - D| = {worst:.3g} eps")
     return ratios
@@ -115,7 +136,24 @@ def test_bound_integer_ties(ctx):
     _check_bound(ctx, X, gb, op, oi, "integer data")
 
 
-def _check_left_out(ctx, X, label, eps_coef, rmax, q, c):
+@pytest.mark.parametrize("d", [64, 128, 200, 384, 768])
+def test_bound_held_exactly(ctx, d):
+    """11-bit significands over seven powers of two, which fp16 holds: the half operands' bound
+    has no rounding term, so the accumulation of the products alone meets it."""
+    rng = np.random.default_rng(400 + d)
+    sizes = rng.choice([3, 40, 200, 700], size=30)
+    gb, op, oi = _random_lng(rng, sizes)
+    shape = (int(gb[-1]), d)
+    X = (rng.integers(-2047, 2048, size=shape) * 2.0 ** rng.integers(-6, 1, size=shape)).astype(np.float32)
+    _check_bound(ctx, X, gb, op, oi, f"held exactly d={d}")
+    coef, lin, _, half = ctx.debug_error_bound()
+    assert lin == 0.0
+    # the half bound's terms: at most 17/16 n u |h(x)||h(q)| of accumulation, 32 u r^2 of the rest
+    hp = (d + 63) // 64 * 64
+    assert not half or coef == pytest.approx((0.6 * hp + 32) * 2.0 ** -24, rel=1e-12)
+
+
+def _check_left_out(ctx, X, label, q, c, operands=None):
     """Every candidate of a partial row's split that the row does not hold (the query
     itself aside) has an exact distance >= bound - eps: exact distances of whole groups
     from fp64 Gram matrices.  Rows of multi-range unions are skipped."""
@@ -124,6 +162,7 @@ def _check_left_out(ctx, X, label, eps_coef, rmax, q, c):
     one = b0 != 0xFFFFFFFF
     Xd = X.astype(np.float64)
     qn32 = (Xd * Xd).sum(axis=1).astype(np.float32).astype(np.float64)
+    eps_all = _eps(ctx, np.sqrt(qn32 * (1.0 + 1e-6)), operands)
     held = {}
     for qq, cc in zip(q.tolist(), c.tolist()):
         held.setdefault(qq, []).append(cc)
@@ -147,7 +186,7 @@ def _check_left_out(ctx, X, label, eps_coef, rmax, q, c):
                         mask[cc - lo] = False
                 if not mask.any() or not np.isfinite(bd[r]):
                     continue
-                eps = eps_coef * (np.sqrt(qn32[qq] * (1.0 + 1e-6)) + rmax) ** 2
+                eps = eps_all[qq]
                 # (bound - D) / eps must stay below 1 (D from a Gram matrix: fp64
                 # cancellation far below eps)
                 v = float((float(bd[r]) - D[j][mask].min()) / eps)
@@ -155,27 +194,29 @@ def _check_left_out(ctx, X, label, eps_coef, rmax, q, c):
                 checked += 1
                 assert v <= 1.0, (f"{label}: query {qq}, split [{lo}, {hi}): a left-out candidate has exact "
                                   f"distance {D[j][mask].min():.9g} < bound {bd[r]:.9g} - eps")
-    _say(f"{label}: {checked} rows' left-out candidates checked, (bound - min D) / eps max {worst:.3g}")
+    _say(f"{label} ({ctx.operands}): {checked} rows' left-out candidates checked, (bound - min D) / eps max {worst:.3g}")
     return checked
 
 
 def _check_group(ctx, X, begins, sizes, K, label):
     ctx.prepare_vectors(X)
     st = ctx.group_knn_device(begins, sizes, K)
-    q, c, a, eps_coef, rmax = ctx.debug_partial_rows()
+    q, c, a, _, _ = ctx.debug_partial_rows()
     assert q.size > 0, f"{label}: no partial-row entries"
+    # lists of fewer than 32 entries below d = 512 keep the split operands
+    operands = ctx.operands if K >= 32 or X.shape[1] >= 512 else "split"
     Xd = X.astype(np.float64)
     qn32 = (Xd * Xd).sum(axis=1).astype(np.float32).astype(np.float64)
     dexact = ((Xd[q.astype(np.int64)] - Xd[c.astype(np.int64)]) ** 2).sum(axis=1)
-    eps = eps_coef * (np.sqrt(qn32[q.astype(np.int64)] * (1.0 + 1e-6)) + rmax) ** 2
+    eps = _eps(ctx, np.sqrt(qn32[q.astype(np.int64)] * (1.0 + 1e-6)), operands)
     r = np.abs(a.astype(np.float64) - dexact) / eps
     # group jobs hold the query's own group only, without the query itself
     grp = np.searchsorted(begins.astype(np.int64), q.astype(np.int64), side="right") - 1
     assert (c.astype(np.int64) >= begins[grp]).all() and (c.astype(np.int64) < begins[grp] + sizes[grp]).all()
     assert not (q == c).any(), f"{label}: a partial row holds its own query"
-    _say(f"{label}: {q.size} entries, rescanned rows {st['fallback_rows']}, |a - D| / eps max {r.max():.3g}")
+    _say(f"{label} ({operands}): {q.size} entries, rescanned rows {st['fallback_rows']}, |a - D| / eps max {r.max():.3g}")
     assert r.max() <= 1.0, f"{label}: |a - D| = {r.max():.3g} eps"
-    assert _check_left_out(ctx, X, label, eps_coef, rmax, q, c) > 0
+    assert _check_left_out(ctx, X, label, q, c, operands) > 0
 
 
 def test_group_bound_cfg2_mid_groups(ctx):
@@ -231,9 +272,9 @@ def test_cross_left_out_single_targets(ctx, d):
     X = (centres[rng.integers(0, 6, size=N)] + 0.05 * rng.standard_normal((N, d))).astype(np.float32)
     ctx.prepare_vectors(X)
     st = ctx.cross_topk_device(gb, op, oi, 6)
-    q, c, _, eps_coef, rmax = ctx.debug_partial_rows()
+    q, c, _, _, _ = ctx.debug_partial_rows()
     _say(f"single targets d={d}: rescanned rows {st['fallback_rows']}")
-    assert _check_left_out(ctx, X, f"single targets d={d}", eps_coef, rmax, q, c) >= 2450 * 3
+    assert _check_left_out(ctx, X, f"single targets d={d}", q, c) >= 2450 * 3
 
 
 def test_debug_rows_refused_without_partial_rows(ctx):
@@ -246,6 +287,8 @@ def test_debug_rows_refused_without_partial_rows(ctx):
         ctx.debug_partial_rows()
     with pytest.raises(F.UngHipError):
         ctx.debug_partial_bounds()
+    with pytest.raises(F.UngHipError):
+        ctx.debug_error_bound()
     ctx.group_knn_device(np.array([0], np.uint32), np.array([300], np.uint32), 8)
     q, _, _, _, _ = ctx.debug_partial_rows()
     assert q.size == 300 * 12  # list_k = 8: 12 entries a row, every one a real candidate
