@@ -343,6 +343,9 @@ def main():
     wall = time.perf_counter() - t0
     ms_per_step = wall * 1e3 / steps
     log(f"{steps} timed steps: {ms_per_step:.3f} ms/step")
+    # the timed cross calls' operands: fp16 (one product a coordinate pair), or bf16 pairs
+    # (three) for a base set or a call that the fp16 ones cannot serve
+    half = ctx.debug_error_bound()[3] and all(s["select_launches"] == 1 for s in cross_stats)
 
     # the drop-in calls with host output (D2H included), after the timed region: the cross
     # rows with distances and sizes, the FlatId rows alone (the reference's flat writeback,
@@ -374,14 +377,14 @@ def main():
     sel_cross_ms = avg(cross_stats, "select_ms")
     sel_intra_ms = avg(intra_stats, "select_ms")
     d = cfg.dim
-    dp = (d + 63) // 64 * 64  # dimensions of an operand row
-    # The cross select kernel's two floors: its MFMA work (one fp16 product per
-    # coordinate pair: 2 * dp flops per algorithmic pair, against the dense 16-bit peak) and its
+    dp = (d + 63) // 64 * 64 if half else (d + 31) // 32 * 32  # dimensions of an operand row
+    # The cross select kernel's two floors: its MFMA work (one fp16 product, or three bf16
+    # ones, per coordinate pair of 2 flops, against the dense 16-bit peak) and its
     # HBM traffic (measured with rocprofv3 on this kernel source, against 8 TB/s).  The
     # larger floor bounds it; without a valid traffic measurement the MFMA floor is used.
     sel_s = sel_cross_ms * 1e-3
     flops_cross = 2.0 * d * p_cross
-    mfma_flops = 2.0 * dp * p_cross
+    mfma_flops = (2.0 if half else 6.0) * dp * p_cross
     alg_bytes = float(cross_stats[-1]["select_bytes"])
     traffic, traffic_status = read_traffic(cfg.name) if not args.n else (None, "not measured (scaled run)")
     mfma_floor_ms = mfma_flops / (MFMA_16BIT_PEAK_TFLOPS * 1e12) * 1e3
@@ -395,8 +398,8 @@ def main():
         roofline = {"bound": "mfma", "achieved": round(mfma_tflops, 3), "peak": MFMA_16BIT_PEAK_TFLOPS,
                     "unit": "TFLOP/s", "frac": round(mfma_tflops / MFMA_16BIT_PEAK_TFLOPS, 4), "traffic": traffic}
     roofline.update({
-        "kernel": ("ung_select_kernel<8,*,false,2,true,true> (cross edges, register-query layout, one launch per step)"
-                   if dp == 128 else "ung_select_kernel<8,*,false,2,false,true> (cross edges, one launch per step)"),
+        "kernel": f"ung_select_kernel<8,*,false,2,{str(dp == 128).lower()},{str(half).lower()}> (cross edges, "
+                  + ("register-query layout, " if dp == 128 else "") + "one launch per step)",
         "avg_launch_ms": round(sel_cross_ms, 4),
         "traffic_status": traffic_status,
         "streamed_operand_bytes_per_launch": alg_bytes,
@@ -411,7 +414,7 @@ def main():
         "metric": METRIC, "value": value, "unit": "distance evals/s", "n_gpus": 1,
         "steps": steps, "warmup": warmup, "ms_per_step": round(ms_per_step, 3),
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-        "dtype": "f32 (certified fp16 MFMA pre-select, exact f32 re-score)",
+        "dtype": f"f32 (certified {'fp16' if half else '3xbf16'} MFMA pre-select, exact f32 re-score)",
         "data": "synthetic",
         "config": {"workload": f"{cfg.name}: {cfg.n}x{cfg.dim} fp32 Gaussian mixture "
                                f"({cfg.n_centroids} centroids, sigma {cfg.sigma}), vocab {cfg.vocab}, "

@@ -13,8 +13,8 @@
 //                       v_mfma_f32_32x32x16_f16 product; the certificate carries the
 //                       largest rounding error the base set really has.  A third of the
 //                       matrix work and half the operand bytes of the split (cross select
-//                       1M x 128 14.2 -> 9.0 ms, 1M x 384 15.5 -> 8.5 ms, 2M x 768 160 ->
-//                       80 ms);
+//                       1M x 128 13.7 -> 8.4 ms, 1M x 384 15.5 -> 8.1 ms, 2M x 768 160 ->
+//                       77 ms, with the items in runs 72 ms);
 //               split : bf16 hi + lo of every coordinate, products hi*hi + hi*lo + lo*hi by
 //                       three v_mfma_f32_32x32x16_bf16 passes: an error bound 3 to 11 times
 //                       smaller.  For base sets outside the half operands' range, and for
@@ -1103,8 +1103,10 @@ __global__ __launch_bounds__(select_threads<NB>(), (LT <= 8 ? 2 : 1)) void ung_s
             // m4-th entries (4*m4 >= Lp+1 entries in all), so a candidate at or above that
             // value is not among the query's Lp+1 best.  The other wave's value is from the
             // previous tile: entries only decrease, so it bounds the current one.  (For
-            // k = 6, Lp = 10: the larger of the four queues' 3rd entries, near the query's
-            // 16th best, against about its 26th for the smallest of their 8th entries.)
+            // k = 6 on half operands, Lp = 16: the largest of the four queues' 5th entries,
+            // at or past the query's 20th best; on split ones, Lp = 10: of their 3rd
+            // entries, near its 16th best, against about its 26th for the smallest of the
+            // 8th entries.)
             float tsh[NB], ncth[NB];
             [[maybe_unused]] float pm4[NB];
 #pragma unroll

@@ -644,23 +644,21 @@ int launch_knn_select_t(ung_hip_ctx *ctx, hipStream_t stream, const SelectParams
 
 int launch_knn_select(ung_hip_ctx *ctx, hipStream_t stream, const SelectParams &P, uint32_t n_items, bool half)
 {
-    switch (P.dp / KC * (half ? 10u : 1u)) {
-    case 10:
+    const uint32_t nk = P.dp / KC; // chunks of an operand row, 64 (half) or 32 dimensions each
+    if (half && nk == 1)
         return launch_knn_select_t<1, true>(ctx, stream, P, n_items);
-    case 20:
+    if (half && nk == 2)
         return launch_knn_select_t<2, true>(ctx, stream, P, n_items);
-    case 1:
+    if (!half && nk == 1)
         return launch_knn_select_t<1, false>(ctx, stream, P, n_items);
-    case 2:
+    if (!half && nk == 2)
         return launch_knn_select_t<2, false>(ctx, stream, P, n_items);
-    case 3:
+    if (!half && nk == 3)
         return launch_knn_select_t<3, false>(ctx, stream, P, n_items);
-    case 4:
+    if (!half && nk == 4)
         return launch_knn_select_t<4, false>(ctx, stream, P, n_items);
-    default:
-        set_error("filter-and-buffer select: operand rows of %u words", P.dp);
-        return UNG_HIP_EINVAL;
-    }
+    set_error("filter-and-buffer select: operand rows of %u words", P.dp);
+    return UNG_HIP_EINVAL;
 }
 
 // Error factor of the expansion-form value a = fl(|q|^2 - 2*acc) of the select kernel on the
@@ -774,8 +772,9 @@ int workspace_mem(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, R
 }
 
 // Copies a plan's jobs and segments into the staging buffer, and its items in order of
-// decreasing cost (candidate tiles): a stable counting sort by tile count (the query
-// blocks of one split stay next to each other).  Large plans run on the worker pool:
+// decreasing cost (candidate tiles): a stable counting sort by tile count (items of one tile
+// count keep the plan's order: the query blocks of one split, or with fine splits the splits
+// of one query block, but an uneven last split goes with the items of its own count).  Large plans run on the worker pool:
 // per-chunk histograms, a prefix over (bucket, chunk), a scatter.
 void stage_plan(ung_hip_ctx *ctx, const Plan &pl, const StageLayout &L, char *hs)
 {
@@ -857,8 +856,8 @@ size_t merge_qlds_bytes(uint32_t d)
 // A half pre-selection that leaves more than one row in HALF_RETRY uncertified (and more
 // than HALF_RETRY_MIN, below which the rescan takes less than another launch) is repeated on
 // the split operands before the rescan.  The exact rescan handles about 2.3e9 pairs/s at
-// d = 128 (cfg2: 14,060 rows of 27,400 candidates, 170 ms), the split select 1.4e12
-// (20.6e9 pairs, 14.4 ms): repeating pays from about one row in 600 on.
+// d = 128 (cfg2: 14,060 rows of 27,400 candidates, 170 ms), the split select 1.5e12
+// (20.6e9 pairs, 13.7 ms): repeating pays from about one row in 650 on.
 constexpr uint32_t HALF_RETRY = 512;
 constexpr uint32_t HALF_RETRY_MIN = 256;
 

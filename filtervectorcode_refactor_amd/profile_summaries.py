@@ -4,10 +4,10 @@
       <dir>/trace/t_kernel_stats.csv, t_kernel_trace.csv and <dir>/trace.log (the bench
       line) of `rocprofv3 --kernel-trace --stats ... -- python3 bench.py --config <config>
       --steps S --warmup 1 --no-cpu-baseline`  ->  profiles/select_<config>_kernel_trace.md
-  python -m filtervectorcode_refactor_amd.profile_summaries counters <dir>
+  python -m filtervectorcode_refactor_amd.profile_summaries counters <config> <dir>
       <dir>/pmc_{A,B,C}/p_counter_collection.csv of three `rocprofv3 --pmc` passes over
-      `bench.py --config cfg2 --steps 1 --warmup 0 --no-cpu-baseline`
-      ->  profiles/select_cfg2_counters.md
+      `bench.py --config <config> --steps 1 --warmup 0 --no-cpu-baseline`
+      ->  profiles/select_<config>_counters.md
   python -m filtervectorcode_refactor_amd.profile_summaries traffic <config> <dir>
       <dir>/{FETCH_SIZE,WRITE_SIZE}/p_counter_collection.csv of two `rocprofv3 --pmc`
       passes over `bench.py --config <config> --steps 1 --warmup 0 --no-cpu-baseline
@@ -98,14 +98,17 @@ def trace(cfg: str, d: str):
     print("wrote", path)
 
 
-def counters(d: str):
+def counters(cfg: str, d: str):
     import bench
+    from filtervectorcode_refactor_amd import datasets as D
+    C = D.CONFIGS[cfg]
     data = collections.OrderedDict()
     for p in "ABC":
         rows = list(csv.DictReader(open(os.path.join(d, f"pmc_{p}", "p_counter_collection.csv"))))
-        for key, label in (("ung_select_kernel<8", "cross select"), ("ung_knn_select_kernel", "intra select"),
-                           ("ung_merge_kernel<false>", "merge")):
-            hit = [r for r in rows if key in r["Kernel_Name"]]
+        for keys, label in ((("ung_select_kernel<8",), "cross select"),
+                            (("ung_knn_select_kernel", "ung_select_kernel<32"), "intra select"),
+                            (("ung_merge_kernel<false>",), "merge")):
+            hit = [r for r in rows if any(key in r["Kernel_Name"] for key in keys)]
             first = min(int(r["Dispatch_Id"]) for r in hit)
             e = data.setdefault(label, {"name": _short(hit[0]["Kernel_Name"]), "dur": {}, "disp": {}})
             for r in hit:
@@ -114,12 +117,12 @@ def counters(d: str):
                     e["dur"][p] = (int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e6
                     e["disp"][p] = first
     cols = list(data)
-    out = ["# Counters — cfg2 (1,000,000 x 128): cross select, intra (mid-group) select, merge; MI355X", "",
+    out = [f"# Counters — {cfg} ({C.n:,} x {C.dim}): cross select, intra (mid-group) select, merge; MI355X", "",
            "Commands (repository root, MI355X box; one counter block per run; the first dispatch of each",
            "kernel in the run; counter collection serializes the dispatches, so each kernel ran alone):", ""]
     for p, cs in PASSES.items():
-        out.append(f"    rocprofv3 --pmc {cs} --output-format csv -d gpurun_out/meas/cfg2/pmc_{p} -o p -- \\")
-        out.append("        python3 bench.py --config cfg2 --steps 1 --warmup 0 --no-cpu-baseline")
+        out.append(f"    rocprofv3 --pmc {cs} --output-format csv -d gpurun_out/meas/{cfg}/pmc_{p} -o p -- \\")
+        out.append(f"        python3 bench.py --config {cfg} --steps 1 --warmup 0 --no-cpu-baseline")
     out += ["", "| counter | " + " | ".join(f"{c} `{data[c]['name']}`" for c in cols) + " |",
             "|---|" + "---:|" * len(cols)]
     names = sorted({k for c in cols for k in data[c] if k.isupper() or k.startswith("SQ_") or k.startswith("TCC") or
@@ -156,7 +159,7 @@ def counters(d: str):
     row("wave cycles waiting (any instruction)", lambda e: f"{e['SQ_WAIT_INST_ANY'] / e['SQ_WAVE_CYCLES'] * 100:.1f} %")
     row("L2 hit rate (TCC)", lambda e: f"{e['TCC_HIT'] / (e['TCC_HIT'] + e['TCC_MISS']) * 100:.1f} %")
     out += ["", f"kernel_source_sha256: {bench.kernel_source_digest()}"]
-    path = os.path.join(ROOT, "profiles", "select_cfg2_counters.md")
+    path = os.path.join(ROOT, "profiles", f"select_{cfg}_counters.md")
     open(path, "w").write("\n".join(out) + "\n")
     print("wrote", path)
 
@@ -211,7 +214,7 @@ if __name__ == "__main__":
     if what == "trace":
         trace(sys.argv[2], sys.argv[3])
     elif what == "counters":
-        counters(sys.argv[2])
+        counters(sys.argv[2], sys.argv[3])
     elif what == "traffic":
         traffic(sys.argv[2], sys.argv[3])
     else:

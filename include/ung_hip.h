@@ -63,7 +63,9 @@ typedef struct ung_hip_stats {
     uint64_t select_bytes;   /* operand bytes the select kernel(s) stream: per work item,
                                 its query rows and its candidate rows of the operand set
                                 (fp16: 2 bytes a coordinate, dim rounded up to 64; split
-                                bf16 pairs: 4 bytes, dim rounded up to 32) */
+                                bf16 pairs: 4 bytes, dim rounded up to 32); of a call
+                                repeated on the split operands, and so padded_pairs: both
+                                selects, the first as far as it ran */
     uint64_t allocations;    /* device (hipMalloc) and pinned host (hipHostMalloc)
                                 allocations the call made (buffers grown on demand) */
 } ung_hip_stats;
@@ -131,7 +133,9 @@ int ung_hip_cross_result_device(ung_hip_ctx *ctx, uint32_t **ids_dev, float **di
  * and flags live in a file-scope device array of UNG_HIP_NOALLOC_SCRATCH_BYTES (64 MiB)
  * per GPU, held until the process ends; a call whose plan needs more returns
  * UNG_HIP_EINVAL (the message gives the bytes needed) -- roughly 600k result rows with
- * single-split unions at k = 6 and d < 512.  The call makes no hipMalloc, hipHostMalloc
+ * single-split unions at k = 6 and d < 512.  From about 0.46M of them on the plan fits only
+ * with the split-bf16 pre-selection's shorter partial rows, and its select takes about 1.7
+ * times as long (1M x 128: 13.7 against 8.4 ms).  The call makes no hipMalloc, hipHostMalloc
  * or hipFree (ung_hip_stats::allocations stays 0); its host work lists reuse the
  * context's storage.  It needs the base set prepared beforehand (ung_hip_prepare_vectors,
  * which allocates, at set-up).  Calls on one GPU share that GPU's array: a per-device
