@@ -75,6 +75,18 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+// What a select knows of its rows' certificates (half operands; count_uncertifiable).  Behind
+// the item counters in device memory, not among the launch's arguments: these stay in scalar
+// registers from the first instruction on, and 10 to 30 more of them spilled (1 to 2 % of the
+// selects of short items).
+struct GiveUp {
+    uint32_t count;       // rows seen that will not be certified, weighted
+    uint32_t taken;       // items taken when the select gave up
+    uint32_t limit;       // past it the blocks take no further items
+    float coef, lin, rmax; // the certificate's error bound (bound_ea), in fp32 for this estimate
+    float most;           // its largest value (|q| = rmax)
+};
+
 struct SelectParams {
     const uint32_t *xs; // pre-selection operands: [N][dp] words, the half or the split base set
                         // (ung_operands_kernel)
@@ -91,12 +103,9 @@ struct SelectParams {
     float *part_dist;
     float *part_bound;
     uint32_t n_items; // items of this launch
-    uint32_t *item_ctr; // next item to take: one counter, or one per XCD (zeroed before the launch)
+    uint32_t *item_ctr; // N_XCD words: next item to take (the first, or one per XCD), zeroed before
+                        // the launch; then the GiveUp of the call
     uint32_t run_log2;  // log2 of the consecutive items one XCD takes (XCD_RUN_NONE: one counter)
-    uint32_t *give_up;  // half operands: [0] rows seen that will not be certified, weighted
-                        // (uncertifiable), [1] items taken when the select gave up
-    uint32_t give_limit; // more than this in [0]: the blocks take no further items
-    float eps_coef, eps_lin, rmax; // the certificate's error bound (bound_ea), in fp32 for this estimate
     uint32_t lp;      // entries per partial row (approximate top-Lp)
     uint32_t x_bytes; // bytes of the split base set (buffer range of the 32-bit-offset kernels)
 };
@@ -501,14 +510,15 @@ __device__ __forceinline__ uint32_t take_item_run(uint32_t *ctr, uint32_t run_lo
 
 // Half operands: a call that leaves too many rows uncertified is repeated on the split
 // operands, so its select counts the rows that the merge will not certify, and past
-// P.give_limit it gives up: the item counters step past the end of the list, no block takes a
+// its limit it gives up: the item counters step past the end of the list, no block takes a
 // further item, and the merge exits on the same count (some partial rows are unwritten).  On
 // data off the origin, against a whole half select and merge and against the split operands
 // alone: lists of 32 at 300k x 128 2.7 -> 1.05 ms (0.85), cross 1M x 128 38.5 -> 25.0 ms
 // (22.7), 78k x 100, k = 10 1.85 -> 1.4 ms (1.0), 300k x 384 13.6 -> 13.0 ms (10.5: its first
-// 512 items take as long as the rest).  Where they certify the rows: 1M x 128 select 8.45 ->
-// 8.47 ms, lists at 300k x 384 0.638 -> 0.647 ms.  Looking at the count within an item as well
-// gave 1M 24.4 and 300k x 384 12.4 ms, and cost every select 1 %.
+// 512 items take as long as the rest).  Where they certify the rows the calls take the same
+// time within 0.5 % (1M x 128, 1M x 384 with its 90k short items, lists at 300k x 384).
+// Looking at the count within an item as well gave 1M 24.4 and 300k x 384 12.4 ms, and cost
+// every select 1 %.
 //
 // uncertifiable: whether the merge will leave a row uncertified, as far as its approximate
 // distances tell: dk its k-th one, A the bound of the candidates left out, qn = |q|^2, all
@@ -517,24 +527,34 @@ __device__ __forceinline__ uint32_t take_item_run(uint32_t *ctr, uint32_t run_lo
 // with a tie at dk (more copies of one vector in this split than the row is long).  The merge
 // alone decides what is certified; this decides only how soon a call gives up.
 constexpr uint32_t GIVE_UNSPLIT = 16;
-__device__ __forceinline__ bool uncertifiable(const SelectParams &P, bool unsplit, float dk, float A, float qn)
+__device__ __forceinline__ GiveUp *give_up_of(const SelectParams &P)
 {
-    const float r = sqrtf(fmaxf(qn, 0.0f)) + P.rmax;
-    return dk < INFINITY && !(A - (P.eps_coef * r + P.eps_lin) * r > dk) && (unsplit || A != dk);
+    return reinterpret_cast<GiveUp *>(P.item_ctr + N_XCD);
+}
+// most: GiveUp::most, loaded ahead of the item's last steps (an item of one tile takes a few
+// microseconds, a load one); what the few rows near it need besides is loaded for them.
+__device__ __forceinline__ bool uncertifiable(const SelectParams &P, float most, const Item &it, float dk, float A,
+                                              float qn)
+{
+    if (A - most > dk || !(dk < INFINITY))
+        return false;
+    const GiveUp *const g = give_up_of(P);
+    const float r = sqrtf(fmaxf(qn, 0.0f)) + g->rmax;
+    return !(A - (g->coef * r + g->lin) * r > dk) && (P.jobs[it.job].n_split == 1u || A != dk);
 }
 
 // One thread a wave adds the wave's count; the one that passes the limit steps the item
-// counters on and leaves the number of items taken so far in P.give_up[1].
-__device__ __forceinline__ void count_uncertifiable(const SelectParams &P, uint32_t n)
+// counters on and leaves the number of items taken so far.
+__device__ __forceinline__ void count_uncertifiable(const SelectParams &P, const Item &it, uint32_t rows)
 {
-    if (n == 0u)
-        return;
-    const uint32_t before = atomicAdd(P.give_up, n);
-    if (before <= P.give_limit && before + n > P.give_limit) {
+    GiveUp *const g = give_up_of(P);
+    const uint32_t n = rows * (P.jobs[it.job].n_split == 1u ? GIVE_UNSPLIT : 1u);
+    const uint32_t before = atomicAdd(&g->count, n);
+    if (before <= g->limit && before + n > g->limit) {
         uint32_t taken = 0u;
         for (uint32_t x = 0; x < (P.run_log2 != XCD_RUN_NONE ? N_XCD : 1u); ++x)
             taken += atomicAdd(P.item_ctr + x, P.n_items);
-        P.give_up[1] = min(taken, P.n_items);
+        g->taken = min(taken, P.n_items);
     }
 }
 
@@ -1438,6 +1458,7 @@ __global__ __launch_bounds__(select_threads<NB>(), (LT <= 8 ? 2 : 1)) void ung_s
     const int npass = qcnt > 64 ? 2 : 1;
     for (int pass = 0; pass < npass; ++pass) {
         const int rows_here = (int)min(64u, qcnt - (uint32_t)pass * 64u);
+        [[maybe_unused]] const float most = HALF ? give_up_of(P)->most : 0.0f;
         __syncthreads();
         // the waves whose query columns lie in this pass's 64 queries
         if ((wn * QW) / 64 == pass) {
@@ -1498,12 +1519,12 @@ __global__ __launch_bounds__(select_threads<NB>(), (LT <= 8 ? 2 : 1)) void ung_s
                 A = fminf(A, sm.u.r.alist[jl][l]);
             P.part_bound[prow] = A * P.inv_s2; // approximate-distance space
             if constexpr (HALF)
-                bad = uncertifiable(P, jb.n_split == 1u, dk * P.inv_s2, A * P.inv_s2, sm.qn[ql] * P.inv_s2);
+                bad = uncertifiable(P, most, it, dk * P.inv_s2, A * P.inv_s2, sm.qn[ql] * P.inv_s2);
         }
         if constexpr (HALF) {
             const uint32_t n_bad = (uint32_t)__popcll(__ballot(bad));
-            if (tid == 0)
-                count_uncertifiable(P, n_bad * (jb.n_split == 1u ? GIVE_UNSPLIT : 1u));
+            if (tid == 0 && n_bad != 0u)
+                count_uncertifiable(P, it, n_bad);
         }
     }
 }
@@ -2051,6 +2072,7 @@ __global__ __launch_bounds__(KNN_THREADS, 1) void ung_knn_select_kernel(SelectPa
 
     // per query (four threads): bitonic sort of its <= KNN_OUT entries by value over
     // elements e = 16p + i, then the partial row and its bound
+    [[maybe_unused]] const float most = HALF ? give_up_of(P)->most : 0.0f;
     __syncthreads();
     {
         const int q = tid >> 2, p = tid & 3;
@@ -2112,10 +2134,10 @@ __global__ __launch_bounds__(KNN_THREADS, 1) void ung_knn_select_kernel(SelectPa
             dk = quad_min(dk);
             const bool bad =
                 p == 0 && (uint32_t)q < qcnt &&
-                uncertifiable(P, jb.n_split == 1u, dk * P.inv_s2, fminf(sm.tau[q], next) * P.inv_s2, sm.qn[q] * P.inv_s2);
+                uncertifiable(P, most, it, dk * P.inv_s2, fminf(sm.tau[q], next) * P.inv_s2, sm.qn[q] * P.inv_s2);
             const uint32_t n_bad = (uint32_t)__popcll(__ballot(bad));
-            if (lane == 0)
-                count_uncertifiable(P, n_bad * (jb.n_split == 1u ? GIVE_UNSPLIT : 1u));
+            if (lane == 0 && n_bad != 0u)
+                count_uncertifiable(P, it, n_bad);
         }
         if ((uint32_t)q < qcnt) {
             const size_t prow = (size_t)jb.part_base + (size_t)it.split * jb.q_count + it.q_off + (uint32_t)q;
@@ -2941,6 +2963,15 @@ __global__ void ung_zero_u32_kernel(uint32_t *p, uint32_t n)
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n)
         p[i] = 0;
+}
+
+// The words of a call's flag array before its select: zero counters, then the GiveUp.
+__global__ void ung_flags_kernel(uint32_t *p, uint32_t n, GiveUp g)
+{
+    if (threadIdx.x < n)
+        p[threadIdx.x] = 0;
+    if (threadIdx.x == 0)
+        *reinterpret_cast<GiveUp *>(p + n) = g;
 }
 
 // Group id (1..G) of every point, from the group-contiguous ranges.

@@ -211,10 +211,9 @@ StageLayout stage_layout(const Plan &pl)
 }
 
 // Words of a call's flag array: rows flagged for the rescan, the select's item counters (one,
-// or one per XCD), and (half operands) the rows it found uncertifiable, the items taken when it
-// gave up.
-constexpr uint32_t FLAG_ROWS = 0, FLAG_ITEMS = 1, FLAG_GIVE_UP = FLAG_ITEMS + N_XCD, FLAG_TAKEN = FLAG_GIVE_UP + 1,
-                   FLAG_WORDS = FLAG_TAKEN + 1;
+// or one per XCD), its GiveUp.
+constexpr uint32_t FLAG_ROWS = 0, FLAG_ITEMS = 1, FLAG_GIVE_UP = FLAG_ITEMS + N_XCD,
+                   FLAG_WORDS = FLAG_GIVE_UP + sizeof(GiveUp) / sizeof(uint32_t);
 
 // Where a planned call reads its work lists, keeps its partial rows and flags, and
 // writes its result rows.
@@ -932,11 +931,17 @@ int plan_launch(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, Pla
 int plan_launch_select(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, PlanMem &m)
 {
     int rc;
-    hipLaunchKernelGGL(ung_zero_u32_kernel, dim3(1), dim3(64), 0, ws.stream, m.flag_count, FLAG_WORDS);
+    const Operands o = operands_of(ctx, m.half);
+    GiveUp g{};
+    g.limit = give_limit(m, pl);
+    g.coef = (float)o.coef;
+    g.lin = (float)o.lin;
+    g.rmax = (float)o.rmax;
+    g.most = (float)((o.coef * 2.0 * o.rmax + o.lin) * 2.0 * o.rmax);
+    hipLaunchKernelGGL(ung_flags_kernel, dim3(1), dim3(64), 0, ws.stream, m.flag_count, FLAG_GIVE_UP, g);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipEventRecord(ws.ev[0], ws.stream));
 
-    const Operands o = operands_of(ctx, m.half);
     const uint32_t lp = m.lp;
     SelectParams P{};
     P.xs = o.xs;
@@ -954,11 +959,6 @@ int plan_launch_select(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t
     P.part_bound = m.part_bound;
     P.item_ctr = m.flag_count + FLAG_ITEMS;
     P.run_log2 = m.half ? item_runs(pl, o.dp, (pl.jobs[0].flags & 1u) != 0) : XCD_RUN_NONE;
-    P.give_up = m.flag_count + FLAG_GIVE_UP;
-    P.give_limit = give_limit(m, pl);
-    P.eps_coef = (float)o.coef;
-    P.eps_lin = (float)o.lin;
-    P.rmax = (float)o.rmax;
     P.lp = lp;
     const uint32_t n_items = (uint32_t)pl.items.size();
     const bool excl = (pl.jobs[0].flags & 1u) != 0; // one kind of job per plan
@@ -1071,7 +1071,10 @@ int plan_finish(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, Pla
     HIPCHECK(hipMemcpyAsync(flags, m.flag_count, sizeof(flags), hipMemcpyDeviceToHost, ws.stream));
     HIPCHECK(hipStreamSynchronize(ws.stream));
     uint32_t nflag = flags[FLAG_ROWS];
-    if (nflag > retry_limit(m, pl) || flags[FLAG_GIVE_UP] > give_limit(m, pl)) {
+    GiveUp g;
+    std::memcpy(&g, flags + FLAG_GIVE_UP, sizeof(g));
+    const bool gave_up = g.count > g.limit;
+    if (nflag > retry_limit(m, pl) || gave_up) {
         if (st) {
             float a = 0, b = 0;
             HIPCHECK(hipEventElapsedTime(&a, ws.ev[0], ws.ev[1]));
@@ -1082,8 +1085,7 @@ int plan_finish(ung_hip_ctx *ctx, Workspace &ws, const Plan &pl, uint32_t k, Pla
             st->select_launches += 1;
             // the items it ran: all, or those at the head of the staged list
             const Item *items = reinterpret_cast<const Item *>(m.stage + stage_layout(pl).oi);
-            const bool gave_up = flags[FLAG_GIVE_UP] > give_limit(m, pl);
-            const uint64_t n = gave_up ? std::min<uint64_t>(flags[FLAG_TAKEN], pl.items.size()) : pl.items.size();
+            const uint64_t n = gave_up ? std::min<uint64_t>(g.taken, pl.items.size()) : pl.items.size();
             st->select_bytes += select_bytes(items, n, operands_of(ctx, m.half).dp);
             for (uint64_t i = 0; i < n; ++i)
                 st->padded_pairs += (uint64_t)BQ * ((items[i].v_end - items[i].v_begin + BC - 1) / BC * BC);
