@@ -5,8 +5,7 @@
   (tests/golden/*_ref.npz, made by tests/golden/make_golden.py): group ranges and LNG rows
   (the reference's trie order), cross ids / distances / sizes, additional edges, every
   intra list (digest) and the stored intra rows -- all bit-exact.
-* cfg3 (1M x 384), cfg4 (2M x 768: its split base set is above 4 GiB, so the wide load
-  mode runs) and cfg5 (10M x 128: above 4 GiB) at full size:
+* cfg3 (1M x 384), cfg4 (2M x 768) and cfg5 (10M x 128) at full size:
   - every cross row: size = min(k, |union|), padding, (dist, id) order, every id inside
     the row's minimum-superset union, and every distance bit-exact against the reference's
     summation order (oracle ungo_l2_pairs, pinned against the compiled reference);
@@ -15,12 +14,15 @@
     multiply-adds, minutes to an hour on the box's CPUs) a random sample of rows,
     bit-exact against the reference's compiled distance + SearchQueue scan (oracle/_ref,
     else the plain-C oracle);
+  - every cross row again on the split operands, whose sets of cfg4 and cfg5 are above 4 GiB
+    (the wide load mode; the half sets are below), equal to the half operands' rows;
   - the additional edges of every group (a random sample when the oracle's scan would
     exceed its budget) against the oracle fed the GPU's cross rows;
   - every intra row (mid groups, K = 32): size, local ids, no self, (dist, id) order,
     distances bit-exact; every group's lists bit-exact against the reference.
 """
 import hashlib
+import os
 
 import numpy as np
 import pytest
@@ -150,6 +152,20 @@ def _full_size(cfg_name, oracle, n_cross_sample, n_intra_groups, addl_budget_dim
     _say(f"{cfg_name} full: {q.size} rows ({rescanned.size} rescanned) against the reference scan")
     res = chk.cross_exact_points(st.base, st.group_begin, pg, st.out_ptr, st.out_idx, q, k)
     _assert_rows_equal(ids[q], dist[q], None, res[0], res[1], None, f"{cfg_name} full cross rows")
+
+    # the same rows on the split operands (cfg4, cfg5: the wide load mode)
+    os.environ["UNG_HIP_NO_HALF"] = "1"
+    try:
+        split = F.HipContext(0)
+    finally:
+        del os.environ["UNG_HIP_NO_HALF"]
+    split.prepare_vectors(st.base)
+    ids2, dist2, size2, stats2 = split.cross_topk(st.group_begin, st.out_ptr, st.out_idx, k)
+    _say(f"{cfg_name} full: split operands, select {stats2['select_ms']:.1f} ms, {stats2['fallback_rows']} rescanned")
+    assert stats2["select_bytes"] > 1.3 * stats["select_bytes"]
+    _assert_rows_equal(ids2, dist2, size2, ids, dist, size, f"{cfg_name} on the split operands")
+    split.close()
+    del ids2, dist2, size2
 
     # additional edges of every group, or a sample within the budget (each group's list depends only on its own
     # cross rows and LNG row, so the oracle gets an LNG with only those rows)
