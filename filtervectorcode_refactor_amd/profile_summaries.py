@@ -71,7 +71,7 @@ def trace(cfg: str, d: str):
     f = rl["mfma_flops_per_launch"]
     out = [f"# Kernel trace — {cfg} ({C.n:,} x {C.dim} fp32, cross k={C.k_cross} + intra K={C.k_intra}), MI355X", "",
            "Command (from the repository root on the MI355X box):", "",
-           f"    rocprofv3 --kernel-trace --stats --output-format csv -d gpurun_out/meas/{cfg}/trace -o t -- \\",
+           f"    rocprofv3 --kernel-trace --stats --output-format csv -d meas/{cfg}/trace -o t -- \\",
            f"        python3 bench.py --config {cfg} --steps {steps} --warmup {warm} --no-cpu-baseline", "",
            "Summary (`t_kernel_stats.csv`; durations in microseconds; the run also holds the drop-in calls",
            "with host output and the parity check after the timed steps):", "",
@@ -121,7 +121,7 @@ def counters(cfg: str, d: str):
            "Commands (repository root, MI355X box; one counter block per run; the first dispatch of each",
            "kernel in the run; counter collection serializes the dispatches, so each kernel ran alone):", ""]
     for p, cs in PASSES.items():
-        out.append(f"    rocprofv3 --pmc {cs} --output-format csv -d gpurun_out/meas/{cfg}/pmc_{p} -o p -- \\")
+        out.append(f"    rocprofv3 --pmc {cs} --output-format csv -d meas/{cfg}/pmc_{p} -o p -- \\")
         out.append(f"        python3 bench.py --config {cfg} --steps 1 --warmup 0 --no-cpu-baseline")
     out += ["", "| counter | " + " | ".join(f"{c} `{data[c]['name']}`" for c in cols) + " |",
             "|---|" + "---:|" * len(cols)]
@@ -182,7 +182,7 @@ def traffic(cfg: str, d: str):
     wc, wk, wd, _, wdisp, _ = read("WRITE_SIZE")
     fs, ws = 1048576.0 / fc, 1048576.0 / wc
     fb, wb = fk * 1024.0 * fs, wk * 1024.0 * ws
-    cmd = ("rocprofv3 --pmc {c} --output-format csv -d gpurun_out/meas/" + cfg + "/{c} -o p -- python3 bench.py "
+    cmd = ("rocprofv3 --pmc {c} --output-format csv -d meas/" + cfg + "/{c} -o p -- python3 bench.py "
            "--config " + cfg + " --steps 1 --warmup 0 --no-cpu-baseline --calib-copy")
     out = f"""HBM traffic of one cross select launch ({_short(name)}), {cfg} {C.n:,} x {C.dim}
 
